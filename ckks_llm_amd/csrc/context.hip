@@ -41,6 +41,9 @@ static u64 half_product_mod(const std::vector<u64>& t, u64 m) {
     return ((r - 1) / 2) % m;
 }
 
+// delta of a prime 2^60 - delta with delta below 2^26 (every T prime of the reference's sets), 0 for any other
+static unsigned pm_delta(u64 m) { return m < (1ull << 60) && (1ull << 60) - m < (1ull << 26) ? (unsigned)((1ull << 60) - m) : 0u; }
+
 static double balanced_double(u64 x, u64 q) { return x > q / 2 ? -(double)(q - x) : (double)x; }
 
 // builds the exact-conversion block "source primes src (pqt indices) -> target primes tgt"
@@ -160,6 +163,10 @@ extern "C" int ckks_ctx_create(ckks_ctx** out, int logN, const uint64_t* p, int 
             if (m < (1ull << 50)) {                                            // FP64 back ends: below 2^41, and the wide one below 2^50
                 twdf[(size_t)i * N + k] = balanced_double(pt[k], m);
                 twdi[(size_t)i * N + k] = balanced_double(it[k], m);
+            } else if (pm_delta(m)) {                                          // the same 8-byte table holds 16 w for the pseudo-Mersenne back end
+                const u64 wf = pt[k] << 4, wi = it[k] << 4;
+                std::memcpy(&twdf[(size_t)i * N + k], &wf, 8);
+                std::memcpy(&twdi[(size_t)i * N + k], &wi, 8);
             }
         }
         ckks::PrimeConst& P = pc[i];
@@ -168,7 +175,7 @@ extern "C" int ckks_ctx_create(ckks_ctx** out, int logN, const uint64_t* p, int 
         P.w1n = it[1]; P.w1n_s = H::shoup(it[1], m);
         P.qd = (double)m; P.qinv_d = 1.0 / (double)m;
         P.n_inv_d = balanced_double(c->n_inv[i], m); P.w1n_d = balanced_double(it[1], m);
-        P.f64_ok = c->f64_ok[i]; P.pad = 0;
+        P.f64_ok = c->f64_ok[i]; P.pm_delta = pm_delta(m);
     }
 
     // ---- reference-named constant tables (host copies; layouts as uploaded at Context_23.cuh:528-701) ----

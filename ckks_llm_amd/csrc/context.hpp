@@ -18,7 +18,7 @@ struct PrimeConst {
     double qd, qinv_d;           // (double)q and 1/q for the FP64 back end
     double n_inv_d, w1n_d;       // balanced representatives of n_inv, w1n as doubles
     int f64_ok;                  // prime small enough for the FP64 back end
-    int pad;
+    unsigned pm_delta;           // q = 2^60 - pm_delta (below 2^26): the pseudo-Mersenne back end runs it; 0 for every other prime
 };
 
 // one block of an exact RNS conversion (BasisConv.cuh:18-58): nsrc source primes -> ntgt target primes
@@ -77,7 +77,7 @@ struct ckks_ctx {
     ckks::PrimeConst* d_primes_moddown = nullptr;   // d_primes with (P/p_i)^-1 folded into the inverse transform's final constants of p_i
     ulonglong2* d_tw_fwd = nullptr;       // [prime][N] (w, shoup(w)), index = reference psi_table index
     ulonglong2* d_tw_inv = nullptr;       // [prime][N] from psiinv_table
-    double* d_twd_fwd = nullptr;          // [prime][N] balanced doubles, FP64 back end (0 entries for large primes)
+    double* d_twd_fwd = nullptr;          // [prime][N] balanced doubles, FP64 back ends; words 16 w for primes 2^60 - delta (pm_delta); 0 for other large primes
     double* d_twd_inv = nullptr;
     ckks::ConvBlock* d_conv = nullptr;    // all conversion blocks
     std::vector<ckks::ConvPlan> plan_pq_to_t, plan_qj_to_t, plan_t_to_pq, plan_hybrid, plan_hybrid_all;   // indexed by level l
@@ -100,7 +100,7 @@ struct ckks_ctx {
     std::vector<DecodeTab> decode_tabs;   // CRT tables of decode_coeffs, one per level, built on first use
     int chain_skew = 0, chain_spin = -1;  // chained transform: limbs a chain's first pass runs ahead of its second (0: default), poll limit of a wait (-1: default)
     void* d_ntt_pair = nullptr;           // completion words of the paired (one-launch, small-batch) transform, one per 128-byte line
-    unsigned pair_resident_blocks[6] = {}; // workgroups of each one-launch kernel that fit the chip at once (occupancy x compute units), by PAIR_KIND_*
+    unsigned pair_resident_blocks[7] = {}; // workgroups of each one-launch kernel that fit the chip at once (occupancy x compute units), by PAIR_KIND_*
     // test / tuning switches (ckks_ctx_set_option): the fused key-switch, rescale and ring-packing launches off; the key switch's
     // last steps as separate launches; conversions into primes below 2^50 in 128-bit integers; the second launch of a transform
     // takes the limbs in forward order; limbs per trip through the inter-pass buffer (0: all)
@@ -123,7 +123,7 @@ int hip_fail(hipError_t e, const char* what);
 // chained (one-launch) transform: tiles left to its finishing launch so far, and the host view of its slot order (for tests)
 int ntt_chain_deferred(ckks_ctx* c, long* tiles);
 // 1 once a paired (one-launch) transform of the context has given up a wait: its output is incomplete and the context unusable
-enum { PAIR_KIND_F64 = 0, PAIR_KIND_WIDE, PAIR_KIND_INT, PAIR_KIND_RESCALE, PAIR_KIND_RESCALE_WIDE, PAIR_KIND_KS_BACK };
+enum { PAIR_KIND_F64 = 0, PAIR_KIND_WIDE, PAIR_KIND_INT, PAIR_KIND_PM, PAIR_KIND_RESCALE, PAIR_KIND_RESCALE_WIDE, PAIR_KIND_KS_BACK };
 int ntt_pair_failed(const ckks_ctx* c);
 int ntt_pair_deferred(ckks_ctx* c, long* tiles, bool stolen = false);        // second-pass tiles that paired launches have left to their limb's last workgroup (synchronises)
 int ntt_extra_forms();                                  // 1 if the library was built with launch forms 2 and 3
@@ -142,6 +142,8 @@ bool ntt_resident_applies(const ckks_ctx* c, int limbs);
 int ntt_resident_round(const ckks_ctx* c);              // limbs per round: one per workgroup of its grid
 // transforms the first `count` of the call's `limbs` limbs (limb order of the two-launch form)
 int launch_ntt_resident(ckks_ctx* c, const NttArgs& args, int limbs, int count, bool inverse);
+// back end of a prime of the context's list: 0 FP64 (q < 2^41), 1 FP64 with a balance per register round (q < 2^50), 2 integer, 3 integer modulo 2^60 - delta
+int ntt_back_end(const ckks_ctx* c, int prime);
 int launch_ntt(ckks_ctx* c, uint64_t* dev, int start_poly_idx, int start_mod_idx, int poly_num, int mod_num,
                int poly_mod_len, long batch_stride_limbs, int batch, bool inverse);
 // Hybrid key switch up to the inverse transform of the two sums, in five launches (four where the input's transform runs as one

@@ -155,7 +155,7 @@ __device__ __forceinline__ void strided_tile(u64* limb, unsigned tile, const typ
         }
         const unsigned counted = claim.start(tid);
         inv_packed<AR, SA, S1>(v, tw, 1u, g, ar);
-        ar.round_end(v);
+        ar.round_end_inv(v);
 #pragma unroll
         for (int j = 0; j < R; j++) lds[(g * R + j) * CW + cl] = v[j];
         __syncthreads();
@@ -251,7 +251,7 @@ __device__ __forceinline__ void row_tile(u64* limb, unsigned tile, const typenam
 #pragma unroll
         for (int j = 0; j < R; j++) v[j] = lrow[padded(u * R + j)];
         inv_packed<AR, SB, S1>(v, tw, tw_off, u, ar);
-        ar.round_end(v);
+        ar.round_end_inv(v);
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < R; j++) lrow[padded(u * R + j)] = v[j];
@@ -602,7 +602,7 @@ static bool pair_applies(const ckks_ctx* c, int limbs, int kind) {
     if (c->ntt_mode == 4 || c->ntt_mode == 5) return true;
     return c->ntt_mode == 0 && limbs <= PAIR_AUTO_LIMBS && pair_blocks(limbs, 16u) <= c->pair_resident_blocks[kind];
 }
-template <class AR> constexpr int pair_kind_of() { return std::is_same<AR, F64Arith>::value ? PAIR_KIND_F64 : std::is_same<AR, F64WideArith>::value ? PAIR_KIND_WIDE : PAIR_KIND_INT; }
+template <class AR> constexpr int pair_kind_of() { return std::is_same<AR, F64Arith>::value ? PAIR_KIND_F64 : std::is_same<AR, F64WideArith>::value ? PAIR_KIND_WIDE : std::is_same<AR, PmArith>::value ? PAIR_KIND_PM : PAIR_KIND_INT; }
 
 template <class AR>
 static int dispatch_logn(ckks_ctx* c, const NttArgs& args, int limbs, bool inverse, bool compact_ok, bool res36_ok = false,
@@ -784,10 +784,24 @@ struct ExtRowArgs {
     const u64* key;              // limb z * key_z_stride + d * key_digit_stride + o
     u64* out;                    // limb z * out_z_stride + o: as an in-place inverse transform leaves it between its passes
     const PrimeConst* primes;
-    const ulonglong2* tw_inv;    // [prime][N]
+    const void* tw_inv;          // [prime][N] in the back end's form
     int ndigits, t_num, blocks, prime0;
     long key_digit_stride, key_z_stride, out_z_stride;
 };
+// Sums of the product phase: 128-bit words and one Barrett reduction for any prime, carry-free sums for primes 2^60 - delta.
+template <class AR> struct ExtSum {
+    u128w a{0, 0};
+    __device__ __forceinline__ void add(u64 x, u64 y) { mac128(a, x, y); }
+    __device__ __forceinline__ void eight(const AR&) {}
+    __device__ __forceinline__ u64 residue(const AR&, const PrimeConst& pr) const { return barrett128(a, pr.q, pr.mu_hi, pr.mu_lo); }
+};
+template <> struct ExtSum<PmArith> {
+    PmSum a;
+    __device__ __forceinline__ void add(u64 x, u64 y) { a.add(x, y); }
+    __device__ __forceinline__ void eight(const PmArith& ar) { a.renormalise(ar); }
+    __device__ __forceinline__ u64 residue(const PmArith& ar, const PrimeConst&) const { return a.reduce(ar); }
+};
+template <class AR>
 __global__ __launch_bounds__(256, 4) void ext_row_fused_kernel(ExtRowArgs a) {
     typedef RowCfg<8, 8> C;
     constexpr int S1 = C::S1, R = C::R, N2 = C::N2, U = C::U, N1 = C::N1, ROWS = C::ROWS;
@@ -802,8 +816,8 @@ __global__ __launch_bounds__(256, 4) void ext_row_fused_kernel(ExtRowArgs a) {
     const unsigned o = blk * (unsigned)a.t_num + t;
     const int prime = a.prime0 + (int)t;
     const PrimeConst& pr = a.primes[prime];
-    const IntArith ar(pr);
-    const ulonglong2* tw = a.tw_inv + (long)prime * N;
+    const AR ar(pr);
+    const typename AR::TW* tw = (const typename AR::TW*)a.tw_inv + (long)prime * N;
     const unsigned u = tid % U, rl = tid / U;
     const unsigned row = tile * ROWS + rl;
     u64* lrow = lds + rl * C::PITCH;
@@ -824,12 +838,10 @@ __global__ __launch_bounds__(256, 4) void ext_row_fused_kernel(ExtRowArgs a) {
         constexpr int H = 2;                                    // loads per chunk; a load's two rows apart = N2 16-byte words
 #pragma unroll 1
         for (int j0 = 0; j0 < ROWS / 2; j0 += H) {
-            u128w acc[2 * H];
+            ExtSum<AR> acc[2 * H];
             ulonglong2 x[H], k[H], xn[H], kn[H];
 #pragma unroll
             for (int j = 0; j < H; j++) {
-                acc[2 * j] = u128w{0, 0};
-                acc[2 * j + 1] = u128w{0, 0};
                 x[j] = cp2[(j0 + j) * N2];
                 k[j] = kp2[(j0 + j) * N2];
             }
@@ -839,25 +851,29 @@ __global__ __launch_bounds__(256, 4) void ext_row_fused_kernel(ExtRowArgs a) {
             }
             for (int d = 0; d < a.ndigits; d += 2) {
 #pragma unroll
-                for (int j = 0; j < H; j++) { mac128(acc[2 * j], x[j].x, k[j].x); mac128(acc[2 * j + 1], x[j].y, k[j].y); }
+                for (int j = 0; j < H; j++) { acc[2 * j].add(x[j].x, k[j].x); acc[2 * j + 1].add(x[j].y, k[j].y); }
                 if (d + 2 < a.ndigits) {
 #pragma unroll
                     for (int j = 0; j < H; j++) { x[j] = cp2[(d + 2) * c_step + (j0 + j) * N2]; k[j] = kp2[(d + 2) * k_step + (j0 + j) * N2]; }
                 }
                 if (d + 1 < a.ndigits) {
 #pragma unroll
-                    for (int j = 0; j < H; j++) { mac128(acc[2 * j], xn[j].x, kn[j].x); mac128(acc[2 * j + 1], xn[j].y, kn[j].y); }
+                    for (int j = 0; j < H; j++) { acc[2 * j].add(xn[j].x, kn[j].x); acc[2 * j + 1].add(xn[j].y, kn[j].y); }
                     if (d + 3 < a.ndigits) {
 #pragma unroll
                         for (int j = 0; j < H; j++) { xn[j] = cp2[(d + 3) * c_step + (j0 + j) * N2]; kn[j] = kp2[(d + 3) * k_step + (j0 + j) * N2]; }
                     }
                 }
+                if ((d & 7) == 6) {                             // eight digits since the sums began or were last renormalised
+#pragma unroll
+                    for (int j = 0; j < 2 * H; j++) acc[j].eight(ar);
+                }
             }
 #pragma unroll
             for (int j = 0; j < H; j++) {
                 u64* srow = lds + (pr0 + 2 * (j0 + j)) * C::PITCH;
-                srow[padded(pu)] = barrett128(acc[2 * j], pr.q, pr.mu_hi, pr.mu_lo);
-                srow[padded(pu + 1)] = barrett128(acc[2 * j + 1], pr.q, pr.mu_hi, pr.mu_lo);
+                srow[padded(pu)] = acc[2 * j].residue(ar, pr);
+                srow[padded(pu + 1)] = acc[2 * j + 1].residue(ar, pr);
             }
         }
     }
@@ -866,14 +882,14 @@ __global__ __launch_bounds__(256, 4) void ext_row_fused_kernel(ExtRowArgs a) {
     u64 v[R];
 #pragma unroll
     for (int j = 0; j < R; j++) v[j] = lrow[padded(u * R + j)];
-    inv_packed<IntArith, 8, S1>(v, tw, tw_off, u, ar);
+    inv_packed<AR, 8, S1>(v, tw, tw_off, u, ar);
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < R; j++) lrow[padded(u * R + j)] = v[j];
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < R; j++) v[j] = lrow[padded(u + j * U)];
-    inv_spread<IntArith, 8, S1, 0>(v, tw, tw_off, ar);
+    inv_spread<AR, 8, S1, 0>(v, tw, tw_off, ar);
     u64* rp = a.out + ((long)z * a.out_z_stride + o) * N + at;
 #pragma unroll
     for (int j = 0; j < R; j++) rp[j * U] = ar.to_mid_inv(v[j]);
@@ -1602,23 +1618,31 @@ int launch_ext_product_inverse_fused(ckks_ctx* c, uint64_t* ext, const uint64_t*
     if (c->ks_split || c->logN != 16 || c->ntt_mode != 0 || c->ev_mid_armed || c->t_num <= 0 || c->gamma <= 0 || c->p_num <= 0) return CKKS_OK;
     if ((((uintptr_t)up | (uintptr_t)swk) & 15u) != 0) return CKKS_OK;                      // the product phase reads 16 bytes at a time
     const int T = c->t_num, prime0 = c->p_num + c->q_num;
-    // the integer back end is what the transforms over T would run on: every T prime too wide for the FP64 forms, or the context set to integers
+    // one integer back end is what the transforms over T would run on: every T prime too wide for the FP64 forms, or the context set to integers
+    const int back_end = ntt_back_end(c, prime0);
     for (int j = 0; j < T; j++)
-        if (c->arith_mode == 0 && c->pqt[prime0 + j] < (1ull << 50)) return CKKS_OK;
+        if (ntt_back_end(c, prime0 + j) != back_end || back_end < 2) return CKKS_OK;
     const int ndigits = (l + 1 + c->p_num - 1) / c->p_num;                                   // cipher_blockNum, ExternalProduct.cuh:87
     if (ndigits > c->dnum) { set_error("external_product_T: the level needs more digits than the key holds (q_num is no multiple of p_num)"); return CKKS_E_INVALID; }
     const int blocks = (c->p_num + l + 1 + c->gamma - 1) / c->gamma;                         // :88
     ExtRowArgs a;
-    a.c = (const u64*)up; a.key = (const u64*)swk; a.out = (u64*)ext; a.primes = c->d_primes; a.tw_inv = (const ulonglong2*)c->d_tw_inv;
+    a.c = (const u64*)up; a.key = (const u64*)swk; a.out = (u64*)ext; a.primes = c->d_primes;
+    a.tw_inv = back_end == 3 ? (const void*)c->d_twd_inv : (const void*)c->d_tw_inv;
     a.ndigits = ndigits; a.t_num = T; a.blocks = blocks; a.prime0 = prime0;
     a.key_digit_stride = (long)T * c->Ri_blockNum; a.key_z_stride = (long)c->Ri_blockNum * T * c->dnum; a.out_z_stride = (long)c->Ri_blockNum * T;
     const int limbs = 2 * blocks * T;
-    hipLaunchKernelGGL(ext_row_fused_kernel, dim3((unsigned)(RowCfg<8, 8>::TILES * limbs)), dim3(256), 0, c->stream, a);
     NttArgs args;
-    args.data = (u64*)ext; args.primes = c->d_primes; args.tw = c->d_tw_inv;
+    args.data = (u64*)ext; args.primes = c->d_primes; args.tw = a.tw_inv;
     args.start_poly_idx = 0; args.start_mod_idx = prime0; args.poly_num = blocks; args.mod_num = T; args.poly_mod_len = T;
     args.batch_stride_limbs = a.out_z_stride; args.limb_base = 0; args.limbs_total = (unsigned)limbs; args.mid = nullptr;
-    hipLaunchKernelGGL((ntt_strided_pass<IntArith, 8, 8, true, false>), dim3(StridedCfg<8, 8>::TILES, limbs), dim3(StridedCfg<8, 8>::THREADS), 0, c->stream, args);
+    const dim3 ge((unsigned)(RowCfg<8, 8>::TILES * limbs)), gs(StridedCfg<8, 8>::TILES, limbs), bs(StridedCfg<8, 8>::THREADS);
+    if (back_end == 3) {
+        hipLaunchKernelGGL(ext_row_fused_kernel<PmArith>, ge, dim3(256), 0, c->stream, a);
+        hipLaunchKernelGGL((ntt_strided_pass<PmArith, 8, 8, true, false>), gs, bs, 0, c->stream, args);
+    } else {
+        hipLaunchKernelGGL(ext_row_fused_kernel<IntArith>, ge, dim3(256), 0, c->stream, a);
+        hipLaunchKernelGGL((ntt_strided_pass<IntArith, 8, 8, true, false>), gs, bs, 0, c->stream, args);
+    }
     CKKS_HIP_TRY(hipGetLastError());
     *done = true;
     return CKKS_OK;
@@ -1642,6 +1666,8 @@ static void pair_resident_blocks(ckks_ctx* c) {
     ask(PAIR_KIND_WIDE, ntt_pair_kernel<F64WideArith, 8, 8, true, false>);
     ask(PAIR_KIND_INT, ntt_pair_kernel<IntArith, 8, 8, false, false>);
     ask(PAIR_KIND_INT, ntt_pair_kernel<IntArith, 8, 8, true, false>);
+    ask(PAIR_KIND_PM, ntt_pair_kernel<PmArith, 8, 8, false, false>);
+    ask(PAIR_KIND_PM, ntt_pair_kernel<PmArith, 8, 8, true, false>);
     ask(PAIR_KIND_RESCALE, rescale_pair_kernel<F64Arith, MidPieces>);
     ask(PAIR_KIND_RESCALE_WIDE, rescale_pair_kernel<F64WideArith, MidLimb>);
     ask(PAIR_KIND_KS_BACK, ks_back_kernel);
@@ -1650,6 +1676,12 @@ static void pair_resident_blocks(ckks_ctx* c) {
 static int launch_ntt_from(ckks_ctx* c, uint64_t* dev, int start_poly_idx, int start_mod_idx, int poly_num, int mod_num,
                            int poly_mod_len, long batch_stride_limbs, int batch, bool inverse, const NttEmbedSource* src,
                            const NttFixedArea* fixed = nullptr);
+
+int ntt_back_end(const ckks_ctx* c, int prime) {
+    if (c->arith_mode != 0) return 2;
+    const u64 m = c->pqt[prime];
+    return m < (1ull << 41) ? 0 : m < (1ull << 50) ? 1 : m < (1ull << 60) && (1ull << 60) - m < (1ull << 26) ? 3 : 2;
+}
 
 int launch_ntt(ckks_ctx* c, uint64_t* dev, int start_poly_idx, int start_mod_idx, int poly_num, int mod_num,
                int poly_mod_len, long batch_stride_limbs, int batch, bool inverse) {
@@ -1678,12 +1710,9 @@ static int launch_ntt_from(ckks_ctx* c, uint64_t* dev, int start_poly_idx, int s
     }
     long limbs = (long)poly_num * mod_num * batch;
     if (limbs > 65535) { set_error("NTT: more than 65535 limbs in one call"); return CKKS_E_INVALID; }
-    // back end per prime: 0 = FP64 (q < 2^41), 1 = FP64 with a balance per register round (q < 2^50), 2 = integer
-    auto klass = [&](int j) {
-        if (c->arith_mode != 0) return 2;
-        const u64 m = c->pqt[start_mod_idx + j];
-        return m < (1ull << 41) ? 0 : m < (1ull << 50) ? 1 : 2;
-    };
+    // back end per prime: 0 = FP64 (q < 2^41), 1 = FP64 with a balance per register round (q < 2^50), 2 = integer, 3 = integer modulo
+    // 2^60 - delta
+    auto klass = [&](int j) { return ntt_back_end(c, start_mod_idx + j); };
     int back_end = klass(0);
     bool mixed = false, compact_ok = true, res36_ok = true;
     for (int j = 0; j < mod_num; j++) {
@@ -1729,6 +1758,10 @@ static int launch_ntt_from(ckks_ctx* c, uint64_t* dev, int start_poly_idx, int s
     if (back_end == 1) {
         args.tw = inverse ? (const void*)c->d_twd_inv : (const void*)c->d_twd_fwd;
         return dispatch_logn<F64WideArith>(c, args, (int)limbs, inverse, false, false, fixed);
+    }
+    if (back_end == 3) {
+        args.tw = inverse ? (const void*)c->d_twd_inv : (const void*)c->d_twd_fwd;
+        return dispatch_logn<PmArith>(c, args, (int)limbs, inverse, false, false, fixed);
     }
     args.tw = inverse ? (const void*)c->d_tw_inv : (const void*)c->d_tw_fwd;
     return dispatch_logn<IntArith>(c, args, (int)limbs, inverse, false, false, fixed);

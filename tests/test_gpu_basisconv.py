@@ -327,3 +327,27 @@ def test_hybrid_keyswitch_and_paired_transform_replayed_from_a_graph():
     assert hip.hipGraphExecDestroy(gexec) == 0 and hip.hipGraphDestroy(graph) == 0
     d.set_stream(None)
     assert hip.hipStreamDestroy(stream) == 0
+
+
+@pytest.mark.parametrize("logN", [12, 13, 16])
+def test_keyswitch_23_with_more_digits_than_a_carry_free_sum_holds(logN):
+    """Ten digits of one prime each over T primes 2^60 - delta: the carry-free sums of the external product are renormalised after eight
+    products.  Key and digits of largest residues among them (q - 1 everywhere), at the top level and at levels of 8, 9 and 2 digits."""
+    q, p, t = CFG2_Q[:10], CFG3_P[:1], REF_PARAMS[16]["t"][:3]
+    pair = Pair(logN, p, q, t, 3)
+    o, d, N = pair.orc, pair.dev, pair.N
+    Q, T, RB, QB, dnum = o.q_num, o.t_num, o.Ri_blockNum, o.Qj_blockNum, o.dnum
+    for largest in (True, False):
+        swk = limbs_uniform(7, t, 2 * dnum * RB, N)
+        if largest:
+            swk[...] = np.array(t, dtype=np.uint64).reshape(1, -1, 1) - 1
+        dswk = to_dev(swk)
+        for l in ((9, 7) if largest else (9, 8, 1)):
+            d2 = np.zeros((Q, N), dtype=np.uint64)
+            d2[:l + 1] = limbs_uniform(30 + l, q[:l + 1], 1, N)[0]
+            wout = np.zeros((2, Q, N), dtype=np.uint64)
+            o.keyswitch_23(wout.reshape(-1), d2.copy().reshape(-1), swk.reshape(-1), l)
+            do = to_dev(np.zeros_like(wout))
+            s1, s2, s3 = DeviceBuffer(8 * N * T * QB), DeviceBuffer(8 * N * T * RB * 2), DeviceBuffer(8 * N * T * RB * 2)
+            d.keyswitch_23(do, to_dev(d2), dswk, l, s1, s2, s3)
+            assert np.array_equal(from_dev(do, wout.shape)[:, :l + 1], wout[:, :l + 1]), (largest, l)

@@ -113,6 +113,33 @@ def test_wide_fp64_backend_at_its_range_ends(logN):
             buf.free()
 
 
+@pytest.mark.parametrize("logN", [8, 11, 12, 13, 14, 15, 16])
+def test_pseudo_mersenne_backend_at_its_range_ends(logN):
+    """Integer butterflies modulo 2^60 - delta: the smallest and the largest delta below 2^26, a T prime of the reference between them, and
+    (in the same call) the first prime past that bound and one far from 2^60, which take the general integer back end; uniform residues
+    and the inputs that drive sums and differences to the ends of their ranges, in both directions, against the oracle."""
+    from ckks_llm_amd.params import small_primes
+    near = small_primes(60, 1 << 17, 40)
+    inside = [m for m in near if (1 << 60) - m < (1 << 26)]
+    assert 3 <= len(inside) < len(near)
+    primes = [inside[0], inside[-1], REF_PARAMS[16]["t"][-1], near[len(inside)], small_primes(55, 1 << 17, 1)[0]]
+    pair = Pair(logN, [], primes)
+    N = pair.N
+    check_fwd_inv(pair, 0, primes, 2, seed=60 + logN, mode=0)
+    for kind in range(4):
+        d = np.empty((1, len(primes), N), dtype=np.uint64)
+        for j, m in enumerate(primes):
+            d[0, j] = (m - 1, np.where(np.arange(N) % 2 == 0, 0, m - 1), np.where((np.arange(N) // 16) % 2 == 0, 1, m - 1),
+                       np.where(np.arange(N) < N // 2, m - 1, 0))[kind]
+        for inverse in (False, True):
+            want = d.copy()
+            (pair.orc.FromNTTInplace if inverse else pair.orc.ToNTTInplace)(want.reshape(-1), 0, 0, 1, len(primes), len(primes))
+            buf = to_dev(d)
+            (pair.dev.FromNTTInplace if inverse else pair.dev.ToNTTInplace)(buf, 0, 0, 1, len(primes), len(primes))
+            assert np.array_equal(from_dev(buf, d.shape), want), (logN, kind, inverse)
+            buf.free()
+
+
 def test_n65536_inter_pass_formats():
     """N = 2^16, FP64 back end: primes below 2^39 take the 5-byte inter-pass buffer, 40-bit primes the in-place 8-byte form, and
     ntt_mode 1 forces the in-place form; all against the oracle.  A batch wider than one launch chunk is not needed: chunks
