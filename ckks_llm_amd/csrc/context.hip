@@ -386,7 +386,7 @@ extern "C" int ckks_ctx_create(ckks_ctx** out, int logN, const uint64_t* p, int 
         if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0) c->cu_count = cus;
         c->device = dev;
         if (rc == CKKS_OK) rc = ckks::ntt_noalloc_init(nullptr);
-        if (rc == CKKS_OK && c->logN == 16) rc = ckks::ntt_pair_init(c);
+        if (rc == CKKS_OK && c->logN >= 13) rc = ckks::ntt_pair_init(c);
     }
     if (rc == CKKS_OK && hipEventCreate(&c->ev0) != hipSuccess) rc = CKKS_E_HIP;
     if (rc == CKKS_OK && hipEventCreate(&c->ev1) != hipSuccess) rc = CKKS_E_HIP;
@@ -466,6 +466,7 @@ extern "C" int ckks_ctx_set_option(ckks_ctx* c, const char* name, long value) {
     else if (n == "conv_int") c->conv_int = value != 0;
     else if (n == "ntt_no_reverse") c->ntt_no_reverse = value != 0;
     else if (n == "pair_no_steal") c->pair_no_steal = value != 0;
+    else if (n == "ntt_fine") { if (value < 0 || value > 4) return CKKS_E_INVALID; c->ntt_fine = (int)value; }
     else if (n == "ntt_chunk") { if (value < 0 || value > 65535) return CKKS_E_INVALID; c->ntt_chunk = (int)value; }
     else { ckks::set_error("ckks_ctx_set_option: unknown name " + n); return CKKS_E_INVALID; }
     return CKKS_OK;

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -100,12 +101,16 @@ struct ckks_ctx {
     std::vector<DecodeTab> decode_tabs;   // CRT tables of decode_coeffs, one per level, built on first use
     int chain_skew = 0, chain_spin = -1;  // chained transform: limbs a chain's first pass runs ahead of its second (0: default), poll limit of a wait (-1: default)
     void* d_ntt_pair = nullptr;           // completion words of the paired (one-launch, small-batch) transform, one per 128-byte line
+    std::vector<hipStream_t> pair_streams;     // streams that have made a paired call of ntt_fine.hip: each has protocol words of its own
+    std::mutex pair_streams_mutex;
+    unsigned fine_pair_blocks[4] = {};         // the same for the paired kernels of ntt_fine.hip, by back end
     unsigned pair_resident_blocks[7] = {}; // workgroups of each one-launch kernel that fit the chip at once (occupancy x compute units), by PAIR_KIND_*
     // test / tuning switches (ckks_ctx_set_option): the fused key-switch, rescale and ring-packing launches off; the key switch's
     // last steps as separate launches; conversions into primes below 2^50 in 128-bit integers; the second launch of a transform
     // takes the limbs in forward order; limbs per trip through the inter-pass buffer (0: all)
     bool ks_split = false, ks_back_split = false, conv_int = false, ntt_no_reverse = false, pair_no_steal = false;
     int ntt_chunk = 0;
+    int ntt_fine = 0;                     // 0: small batches take the forms of ntt_fine.hip by the rule there, 1 .. 3: whole limbs / two passes / paired passes wherever they exist, 4: never
     unsigned* h_pair_fail = nullptr;      // pinned host word that a paired transform raises when one of its waits ran out
     void* d_ntt_chain = nullptr;          // completion words of the chained (one-launch) transform, allocated on its first use; zero between transforms
 };
@@ -138,6 +143,10 @@ int launch_ntt_noalloc(ckks_ctx* c, uint64_t* dev, int start_poly_idx, int start
                        bool inverse);
 // Resident transform (ntt_resident.hip): whether it takes a call of `limbs` limbs, and its launch (FP64 back end, primes below 2^36).
 struct NttArgs;
+// Small batches and rings (ntt_fine.hip): which form a call takes (0: none of them) and its launch.
+void ntt_fine_init(ckks_ctx* c);
+int ntt_fine_form(const ckks_ctx* c, int limbs, int back_end);
+int launch_ntt_fine(ckks_ctx* c, const NttArgs& a, int limbs, bool inverse, int back_end, int form);
 bool ntt_resident_applies(const ckks_ctx* c, int limbs);
 int ntt_resident_round(const ckks_ctx* c);              // limbs per round: one per workgroup of its grid
 // transforms the first `count` of the call's `limbs` limbs (limb order of the two-launch form)

@@ -31,7 +31,7 @@
 
 #include "context.hpp"
 #include "ntt_core.hpp"
-#include "pair_protocol.hpp"
+#include "pair_run.hpp"
 
 namespace ckks {
 
@@ -39,35 +39,6 @@ namespace ckks {
 // ------------------------------------------------------------------------------------------------------------
 // strided pass (first SA forward stages / last SA inverse stages): one tile = CW adjacent columns, all N1 rows
 // ------------------------------------------------------------------------------------------------------------
-
-// The two questions that a workgroup of a paired launch asks of its limb's protocol words (pair_protocol.hpp) with atomics that
-// return an answer - the claim of its own first-pass tile and its counting out - ride inside a tile: lane 0 asks behind the
-// tile's own loads (memory operations return in the order of their issue, so an answer that queues behind the other workgroups'
-// atomics on the same words does not hold the loads up) and publishes the answer in LDS, the claim just ahead of the tile's
-// first barrier, the count at the tile's end.  Behind that barrier every lane knows whether a claimed tile is this workgroup's;
-// up to there a tile only reads global memory and writes LDS, so a tile that turns out to be another's leaves no trace.
-// Default: nothing to ask.
-struct TileClaim {
-    unsigned* lds = nullptr;       // where the answer is published (nullptr: nothing to ask)
-    unsigned* words = nullptr;     // the limb's protocol words
-    unsigned tile = 0;
-    bool counting_out = false;     // false: the claim of a first-pass tile; true: the counting out, inside a second-pass tile
-    // start() only issues the atomic and returns what it will bring, untouched: anything computed from it here would make the
-    // wave wait for it at this point; publish() is where it is first looked at
-    __device__ __forceinline__ unsigned start(unsigned tid) const {
-        unsigned v = 0;
-        if (lds && tid == 0) {
-            asm volatile("" ::: "memory");
-            v = counting_out ? pair::Atomics::fetch_add(words + pair::LEFT, 1u) : pair::Atomics::fetch_or(words + pair::CLAIM, 1u << tile);
-        }
-        return v;
-    }
-    // claim: the tile, or LEAVE if it was taken; counting out: how many had left before (the last one out sees TILES - 1)
-    __device__ __forceinline__ void publish(unsigned tid, unsigned raw) const {
-        if (lds && tid == 0) *lds = counting_out ? raw : ((raw >> tile) & 1u ? pair::LEAVE : tile);
-    }
-    __device__ __forceinline__ bool lost() const { return lds && !counting_out && *lds == pair::LEAVE; }
-};
 
 // PAIRED: the tile is one half of a paired transform - what it hands to or takes from the other pass moves as shared accesses
 template <class AR, int SA, int SB, bool INVERSE, bool COHERENT, bool COMPACT = false, bool EMBED = false, bool PAIRED = false>
@@ -336,91 +307,6 @@ unsigned ntt_chain_slots(unsigned kmax, unsigned tiles, unsigned skew) { return 
 // Blocks are numbered so that the tiles of a limb go to one XCD (workgroup b of a grid goes to XCD b mod 8): the inter-pass
 // data then stays in that XCD's L2.  Placement only matters for speed.
 // ------------------------------------------------------------------------------------------------------------
-constexpr unsigned PAIR_XCDS = 8;
-constexpr int PAIR_MAX_LIMBS = 4096;               // protocol words per context
-constexpr int PAIR_GROUPED_LIMBS = 40;             // ... and up to this many with a limb's tiles on one XCD, above it spread over all
-constexpr int PAIR_WORD_STRIDE = pair::WORDS;      // protocol words per limb (pair_protocol.hpp)
-constexpr int PAIR_AUTO_LIMBS = 128;               // automatic mode: batches up to this many limbs take the paired kernel (while the grid fits the chip)
-struct PairArgs {
-    unsigned* done;            // [limb * PAIR_WORD_STRIDE] the limb's protocol words (pair_protocol.hpp), zero between launches
-    unsigned* fail;            // host-visible word: nonzero once a wait of the key switch's last launch has run out
-    unsigned limbs;
-    unsigned spin_steal;       // polls after which a waiting workgroup takes over tiles whose workgroups have not started
-    unsigned spin_max;         // polls after which it leaves its second-pass tiles to the last workgroup out
-    unsigned steal;            // 0: no workgroup takes over another's tile (a test setting)
-    unsigned spread;           // the tiles of a limb go to consecutive workgroups, i.e. to all XCDs (larger batches, and a test setting)
-};
-// (limb, tile) of workgroup b of a paired launch
-__device__ __forceinline__ void pair_block(const PairArgs& p, unsigned b, unsigned tiles, unsigned& limb_id, unsigned& tile) {
-    const unsigned idx = b / PAIR_XCDS;
-    limb_id = p.spread ? b / tiles : b % PAIR_XCDS + PAIR_XCDS * (idx / tiles);
-    tile = p.spread ? b % tiles : idx % tiles;
-}
-// The two passes of (limb_id, tile) under the protocol.  pass1(t) and pass2(t) run tile t on the whole workgroup (t is the
-// workgroup's own tile unless it has taken over others; uniform over the workgroup).  stealing = false: a workgroup only ever
-// runs its own tile (the first pass is work that only this workgroup can do, already under way when this is called).
-template <class P1, class P2>
-__device__ __forceinline__ void pair_run(const PairArgs& p, unsigned limb_id, unsigned tile, unsigned* sh, bool stealing, P1 pass1, P2 pass2) {
-    static_assert(pair::TILES == 16, "sixteen tiles per limb");
-    unsigned* w = p.done + (size_t)limb_id * PAIR_WORD_STRIDE;
-    // The claim of the own tile travels while the tile's loads do (see TileClaim); a tile taken over later is claimed before it starts.
-    TileClaim own;
-    own.lds = stealing ? sh : nullptr;
-    own.words = w;
-    own.tile = tile;
-    unsigned mine = 0, act = tile;
-    for (bool first = true;; first = false) {
-        pass1(act, first ? own : TileClaim());
-        if (first && own.lost()) { act = pair::LEAVE; break; }                  // uniform: behind the tile's first barrier every lane reads the same word
-        mine |= 1u << act;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_s_waitcnt(0);                                          // every shared store of this wave has been acknowledged
-        __syncthreads();
-        if (threadIdx.x == 0) *sh = pair::tile_done_then_decide(w, stealing, p.spin_steal, p.spin_max);
-        // The deciding lane's LDS write is complete before its wave reaches the barrier: said explicitly, because a barrier in a
-        // loop has been seen compiled with no wait for a write that reaches it over the loop's back edge.
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        act = *sh;
-        __syncthreads();
-        if (act >= pair::TILES) break;
-    }
-    // Counting out does not wait for the own second pass: nothing that the last workgroup out does (the second pass of tiles that
-    // others have left, the reset of the words) depends on it.  It rides inside the first second-pass tile (see TileClaim); a
-    // workgroup with no second pass to run counts out here.
-    unsigned todo = act == pair::GO ? mine : 0u;
-    TileClaim out;
-    out.lds = sh;
-    out.words = w;
-    out.counting_out = true;
-    if (todo == 0u && threadIdx.x == 0) {
-        if (act == pair::DEFER) pair::defer(w, mine);
-        *sh = pair::Atomics::fetch_add(w + pair::LEFT, 1u);
-    }
-    for (bool first = true; todo; first = false) {
-        const unsigned t = (unsigned)__builtin_ctz(todo);
-        todo &= todo - 1u;
-        __syncthreads();                                                        // the tile before is done with the LDS
-        pass2(t, first ? out : TileClaim());
-    }
-    __builtin_amdgcn_s_waitcnt(0xc07f);                                         // lgkmcnt(0) only: the LDS write above, not the tile's last stores
-    __syncthreads();
-    if (*sh + 1u != pair::TILES) return;                                        // how many had counted out before this workgroup
-    // last out: every first-pass tile of the limb is complete; what the others left undone, then the words back to zero
-    __syncthreads();
-    if (threadIdx.x == 0) *sh = pair::Atomics::load(w + pair::TODO) & pair::ALL;
-    __builtin_amdgcn_s_waitcnt(0xc07f);
-    __syncthreads();
-    const unsigned finished = *sh;
-    todo = finished;
-    while (todo) {
-        const unsigned t = (unsigned)__builtin_ctz(todo);
-        todo &= todo - 1u;
-        __syncthreads();
-        pass2(t, TileClaim());
-    }
-    if (threadIdx.x == 0) pair::reset(w, finished);
-}
 template <class AR, int SA, int SB, bool INVERSE, bool COMPACT>
 __global__ __launch_bounds__(256, 4) void ntt_pair_kernel(NttArgs a, PairArgs p) {
     typedef StridedCfg<SA, SB> CS;
@@ -459,12 +345,14 @@ static void pair_resident_blocks(ckks_ctx* c);      // defined behind the kernel
 // Protocol words and failure word of the paired transform, once per context (at its creation, so that no transform allocates).
 int ntt_pair_init(ckks_ctx* c) {
     if (c->d_ntt_pair) return CKKS_OK;
-    if (hipHostMalloc((void**)&c->h_pair_fail, sizeof(unsigned), hipHostMallocMapped) != hipSuccess) { set_error("NTT: cannot allocate the failure word of the paired transform"); return CKKS_E_NOMEM; }
-    *c->h_pair_fail = 0;
+    // the failure word is raised by the key switch's last launch only, which exists at N = 2^16
+    if (c->logN == 16 && hipHostMalloc((void**)&c->h_pair_fail, sizeof(unsigned), hipHostMallocMapped) != hipSuccess) { set_error("NTT: cannot allocate the failure word of the paired transform"); return CKKS_E_NOMEM; }
+    if (c->h_pair_fail) *c->h_pair_fail = 0;
     const size_t bytes = ((size_t)PAIR_MAX_LIMBS + 64) * PAIR_WORD_STRIDE * sizeof(unsigned);      // the last 64: counters of ks_back_kernel
     if (hipMalloc(&c->d_ntt_pair, bytes) != hipSuccess) { set_error("NTT: cannot allocate the completion words of the paired transform"); return CKKS_E_NOMEM; }
     CKKS_HIP_TRY(hipMemset(c->d_ntt_pair, 0, bytes));          // complete before the caller can launch anything on any stream
-    pair_resident_blocks(c);
+    if (c->logN == 16) pair_resident_blocks(c);
+    ntt_fine_init(c);
     return CKKS_OK;
 }
 int ntt_pair_failed(const ckks_ctx* c) { return c->h_pair_fail && *(volatile unsigned*)c->h_pair_fail ? 1 : 0; }
@@ -485,7 +373,7 @@ int ntt_extra_forms() {
 #endif
 }
 
-static PairArgs pair_args(const ckks_ctx* c, int limbs) {
+PairArgs pair_args(const ckks_ctx* c, int limbs) {
     PairArgs p;
     p.done = (unsigned*)c->d_ntt_pair; p.fail = c->h_pair_fail; p.limbs = (unsigned)limbs;
     p.spin_max = c->chain_spin >= 0 ? (unsigned)c->chain_spin : 4000000u;
@@ -494,7 +382,7 @@ static PairArgs pair_args(const ckks_ctx* c, int limbs) {
     p.spread = c->ntt_mode == 5 || (c->ntt_mode == 0 && limbs > PAIR_GROUPED_LIMBS) ? 1u : 0u;
     return p;
 }
-static unsigned pair_blocks(int limbs, unsigned tiles) { return ((unsigned)limbs + PAIR_XCDS - 1) / PAIR_XCDS * PAIR_XCDS * tiles; }
+unsigned pair_blocks(int limbs, unsigned tiles) { return ((unsigned)limbs + PAIR_XCDS - 1) / PAIR_XCDS * PAIR_XCDS * tiles; }
 
 template <class AR, int SA, int SB>
 static int launch_pair(ckks_ctx* c, NttArgs args, int limbs, bool inverse, bool compact_ok, char* mid = nullptr) {
@@ -1750,6 +1638,13 @@ static int launch_ntt_from(ckks_ctx* c, uint64_t* dev, int start_poly_idx, int s
         args.embed_p0 = src->p0; args.embed_q0 = src->q0;
         args.embed_logk = src->logk; args.embed_loggap = src->loggap; args.embed_n1 = src->n1;
         args.embed_no_wrap = src->q0 / 2 < src->p0 ? 1 : 0;
+    }
+    if (!src && !fixed && ((uintptr_t)dev & 15u) == 0) {                  // the fine forms move a lane's words 16 bytes at a time
+        const int form = ntt_fine_form(c, (int)limbs, back_end);
+        if (form) {
+            args.tw = back_end == 2 ? (inverse ? (const void*)c->d_tw_inv : (const void*)c->d_tw_fwd) : (inverse ? (const void*)c->d_twd_inv : (const void*)c->d_twd_fwd);
+            return launch_ntt_fine(c, args, (int)limbs, inverse, back_end, form);
+        }
     }
     if (back_end == 0) {
         args.tw = inverse ? (const void*)c->d_twd_inv : (const void*)c->d_twd_fwd;

@@ -30,6 +30,8 @@ struct IntArith {
     template <int R> __device__ __forceinline__ void round_end(V (&)[R]) const {}          // lazy ranges hold for a whole pass
     template <int R> __device__ __forceinline__ void round_end_inv(V (&)[R]) const {}
     __device__ __forceinline__ void stage_end_inv(V&, int) const {}
+    static constexpr int FWD_STAGES = 64, INV_STAGES = 64;                      // stages between two calls of settle()
+    __device__ __forceinline__ V settle(V x) const { return x; }
     // Harvey lazy butterflies; ranges as ntt_60bit.cuh:293-318
     __device__ __forceinline__ void ct(V& x, V& y, TW w) const {
         x = x >= q2 ? x - q2 : x;
@@ -95,6 +97,8 @@ struct F64Arith {
     template <int R> CKKS_HD void round_end(V (&)[R]) const {}          // q < 2^41: the ranges hold for a whole pass
     template <int R> CKKS_HD void round_end_inv(V (&)[R]) const {}
     CKKS_HD void stage_end_inv(V&, int) const {}
+    static constexpr int FWD_STAGES = 16, INV_STAGES = 8;                       // stages between two calls of settle(): the ranges in ntt.hip
+    CKKS_HD V settle(V x) const { return balance(x); }
     CKKS_HD void ct(V& x, V& y, TW w) const {
         double t = mulmod(y, w);
         y = x - t;
@@ -147,6 +151,7 @@ struct F64WideArith : F64Arith {
         for (int j = 0; j < R; j++) v[j] = balance(v[j]);
     }
     template <int R> CKKS_HD void round_end_inv(V (&v)[R]) const { round_end(v); }
+    static constexpr int FWD_STAGES = 4, INV_STAGES = 4;
     CKKS_HD void gs_last(V& x, V& y, u64& ox, u64& oy) const {
         double s = x + y, d = x - y;
         CKKS_RANGE(value(s, "F64WideArith::gs_last sum"));
@@ -212,6 +217,10 @@ struct PmArith {
     }
     template <int R> CKKS_HD void round_end_inv(V (&)[R]) const {}
     CKKS_HD void stage_end_inv(V& sum, int s) const { if (s % 3 == 1) sum = fold(sum); }
+    // forward: seven stages from a folded value stay below 15.1; inverse rounds of three stages end at 2.14 and may start
+    // there, rounds of four start from a settled value
+    static constexpr int FWD_STAGES = 7, INV_STAGES = 6;
+    CKKS_HD V settle(V x) const { return fold(x); }
     CKKS_HD void ct(V& x, V& y, TW w) const {
         const u64 t = mulmod(y, w);
         y = x + q2 - t;

@@ -1,0 +1,200 @@
+// Line transforms in rounds of at most RL stages: a line (a column or row of the two-pass decomposition, or a whole limb) of 2^S
+// values is spread over 2^(S-RL) lanes that hold R = 2^RL values each, and crosses LDS between rounds.
+//
+// The passes of ntt.hip give a lane sixteen values: at a full chip that is the cheapest form (one exchange per pass), but a call of a
+// few limbs then occupies a fraction of the 1024 SIMDs with one wave each, whose butterflies follow one another (64 per lane and
+// pass, 24 instructions each modulo a 60-bit prime: 3.4 us with nothing beside them).  With eight values a lane has half the
+// chain and the launch twice the waves.
+//
+// Round structure (forward): the first round takes S mod RL stages (RL if that is zero), every later one RL, so the last round ends on
+// 2^RL adjacent values per lane, which leave (or arrive, inverse) in 16-byte accesses without a transposition through LDS.
+// Round at stage offset O with C stages, group G = u + h * (lanes per line): positions hi * 2^(S-O) + j * 2^(S-O-C) + lo with
+// lo = G mod 2^(S-O-C), hi = G / 2^(S-O-C); its twiddles are those of the sub-transform hi of 2^(S-O) points.
+// A lane writes the positions that it read, so one barrier per exchange suffices.
+#pragma once
+#include "pair_run.hpp"
+
+namespace ckks {
+
+template <int S, int RL> constexpr int line_first() { return S % RL ? S % RL : RL; }
+
+template <class AR, int C>
+struct TwSet {
+    typename AR::TW t[(1 << C) - 1];
+    __device__ __forceinline__ void load(const typename AR::TW* __restrict__ tw, unsigned base) {
+#pragma unroll
+        for (int s = 0; s < C; s++)
+#pragma unroll
+            for (int i = 0; i < (1 << s); i++) t[(1 << s) - 1 + i] = tw[(base << s) + i];
+    }
+};
+
+template <int S, int RL, int O, int C>
+struct LineRound {
+    static constexpr int GROUPS = 1 << (RL - C), LB = S - O - C;
+    static __device__ __forceinline__ unsigned group(unsigned u, int h) { return u + (unsigned)h * (1u << (S - RL)); }
+    static __device__ __forceinline__ unsigned hi(unsigned g) { return g >> LB; }
+    static __device__ __forceinline__ unsigned pos(unsigned g, int j) {
+        return ((g >> LB) << (S - O)) | ((unsigned)j << LB) | (g & ((1u << LB) - 1u));
+    }
+};
+
+// the twiddles of one round of a lane's groups
+template <class AR, int S, int RL, int O, int C>
+struct RoundTw {
+    TwSet<AR, C> w[1 << (RL - C)];
+    __device__ __forceinline__ void load(const typename AR::TW* __restrict__ tw, unsigned tw_off, unsigned u) {
+        typedef LineRound<S, RL, O, C> LR;
+#pragma unroll
+        for (int h = 0; h < LR::GROUPS; h++) w[h].load(tw, (tw_off << O) + LR::hi(LR::group(u, h)));
+    }
+};
+
+template <class AR, int RL, int C>
+__device__ __forceinline__ void line_butterflies_fwd(typename AR::V (&v)[1 << RL], const TwSet<AR, C> (&w)[1 << (RL - C)], const AR& ar) {
+#pragma unroll
+    for (int h = 0; h < (1 << (RL - C)); h++)
+#pragma unroll
+        for (int s = 0; s < C; s++) {
+            const int half = (1 << C) >> (s + 1);
+#pragma unroll
+            for (int j = 0; j < (1 << C); j++)
+                if ((j & half) == 0) ar.ct(v[(h << C) + j], v[(h << C) + j + half], w[h].t[(1 << s) - 1 + (j >> (C - s))]);
+        }
+}
+template <class AR, int RL, int C, int STOP>
+__device__ __forceinline__ void line_butterflies_inv(typename AR::V (&v)[1 << RL], const TwSet<AR, C> (&w)[1 << (RL - C)], const AR& ar) {
+#pragma unroll
+    for (int h = 0; h < (1 << (RL - C)); h++)
+#pragma unroll
+        for (int s = C - 1; s >= STOP; s--) {
+            const int half = (1 << C) >> (s + 1);
+#pragma unroll
+            for (int j = 0; j < (1 << C); j++)
+                if ((j & half) == 0) {
+                    ar.gs(v[(h << C) + j], v[(h << C) + j + half], w[h].t[(1 << s) - 1 + (j >> (C - s))]);
+                    ar.stage_end_inv(v[(h << C) + j], s);
+                }
+        }
+}
+
+// Forward: v holds the values of the first round (group h, element j at v[(h << C0) + j], position LineRound<..0, C0>::pos) and on
+// return those of the last round (R adjacent positions R u ..).  DONE: stages since the values were last settled.
+// at(pos): LDS word of a position of this lane's line.
+// claim, raw: in a paired launch, the claim of this first-pass tile, published ahead of the first barrier; false is returned (by every
+// lane, nothing stored in global memory yet) when the tile is another workgroup's.
+__device__ __forceinline__ bool line_barrier(const TileClaim& claim, unsigned raw, bool first) {
+    if (first) claim.publish(threadIdx.x, raw);
+    __syncthreads();
+    return !(first && claim.lost());
+}
+template <class AR, int S, int RL, int O, int C, int DONE, class At>
+__device__ __forceinline__ bool line_fwd_rounds(typename AR::V (&v)[1 << RL], const RoundTw<AR, S, RL, O, C>& w, const typename AR::TW* __restrict__ tw,
+                                                unsigned tw_off, unsigned u, const AR& ar, At at, const TileClaim& claim, unsigned raw) {
+    line_butterflies_fwd<AR, RL, C>(v, w.w, ar);
+    if constexpr (O + C < S) {
+        typedef LineRound<S, RL, O, C> A;
+        typedef LineRound<S, RL, O + C, RL> B;
+        constexpr bool SETTLE = DONE + C + RL > AR::FWD_STAGES;
+        RoundTw<AR, S, RL, O + C, RL> wn;                       // requested ahead of the exchange
+        wn.load(tw, tw_off, u);
+        if constexpr (SETTLE) {
+#pragma unroll
+            for (int j = 0; j < (1 << RL); j++) v[j] = ar.settle(v[j]);
+        }
+#pragma unroll
+        for (int h = 0; h < A::GROUPS; h++)
+#pragma unroll
+            for (int j = 0; j < (1 << C); j++) *at(A::pos(A::group(u, h), j)) = v[(h << C) + j];
+        if (!line_barrier(claim, raw, O == 0)) return false;
+#pragma unroll
+        for (int j = 0; j < (1 << RL); j++) v[j] = *at(B::pos(u, j));
+        return line_fwd_rounds<AR, S, RL, O + C, RL, (SETTLE ? 0 : DONE + C)>(v, wn, tw, tw_off, u, ar, at, claim, raw);
+    }
+    return true;
+}
+template <class AR, int S, int RL, class At>
+__device__ __forceinline__ bool line_fwd(typename AR::V (&v)[1 << RL], const RoundTw<AR, S, RL, 0, line_first<S, RL>()>& w,
+                                         const typename AR::TW* __restrict__ tw, unsigned tw_off, unsigned u, const AR& ar, At at,
+                                         const TileClaim& claim = TileClaim(), unsigned raw = 0) {
+    return line_fwd_rounds<AR, S, RL, 0, line_first<S, RL>(), 0>(v, w, tw, tw_off, u, ar, at, claim, raw);
+}
+
+// Inverse: v holds the R adjacent values R u .. on entry and the values of the first forward round on return, with that round's
+// stage 0 left out when LAST (the caller runs it with N^-1 folded in).
+template <class AR, int S, int RL, int O, int C, int DONE, bool LAST, class At>
+__device__ __forceinline__ bool line_inv_rounds(typename AR::V (&v)[1 << RL], const RoundTw<AR, S, RL, O, C>& w, const typename AR::TW* __restrict__ tw,
+                                                unsigned tw_off, unsigned u, const AR& ar, At at, const TileClaim& claim, unsigned raw) {
+    line_butterflies_inv<AR, RL, C, (LAST && O == 0) ? 1 : 0>(v, w.w, ar);
+    if constexpr (O > 0) {
+        constexpr int CN = O == line_first<S, RL>() ? line_first<S, RL>() : RL;
+        typedef LineRound<S, RL, O, C> A;
+        typedef LineRound<S, RL, O - CN, CN> B;
+        constexpr bool SETTLE = DONE + C + CN > AR::INV_STAGES;
+        RoundTw<AR, S, RL, O - CN, CN> wn;
+        wn.load(tw, tw_off, u);
+        if constexpr (SETTLE) {
+#pragma unroll
+            for (int j = 0; j < (1 << RL); j++) v[j] = ar.settle(v[j]);
+        }
+#pragma unroll
+        for (int h = 0; h < A::GROUPS; h++)
+#pragma unroll
+            for (int j = 0; j < (1 << C); j++) *at(A::pos(A::group(u, h), j)) = v[(h << C) + j];
+        if (!line_barrier(claim, raw, O == S - RL)) return false;
+#pragma unroll
+        for (int h = 0; h < B::GROUPS; h++)
+#pragma unroll
+            for (int j = 0; j < (1 << CN); j++) v[(h << CN) + j] = *at(B::pos(B::group(u, h), j));
+        return line_inv_rounds<AR, S, RL, O - CN, CN, (SETTLE ? 0 : DONE + C), LAST>(v, wn, tw, tw_off, u, ar, at, claim, raw);
+    }
+    return true;
+}
+// w: the twiddles of the last round (stage offset S - RL)
+template <class AR, int S, int RL, bool LAST, class At>
+__device__ __forceinline__ bool line_inv(typename AR::V (&v)[1 << RL], const RoundTw<AR, S, RL, S - RL, RL>& w, const typename AR::TW* __restrict__ tw,
+                                         unsigned tw_off, unsigned u, const AR& ar, At at, const TileClaim& claim = TileClaim(), unsigned raw = 0) {
+    return line_inv_rounds<AR, S, RL, S - RL, RL, 0, LAST>(v, w, tw, tw_off, u, ar, at, claim, raw);
+}
+// stage 0 of a transform's last inverse round with N^-1 folded in: canonical words, o[(h << C0) + j] at the position of v[(h << C0) + j]
+template <class AR, int S, int RL>
+__device__ __forceinline__ void line_inv_last(typename AR::V (&v)[1 << RL], u64 (&o)[1 << RL], const AR& ar) {
+    constexpr int C = line_first<S, RL>(), HALF = (1 << C) / 2;
+#pragma unroll
+    for (int h = 0; h < (1 << (RL - C)); h++)
+#pragma unroll
+        for (int j = 0; j < HALF; j++) ar.gs_last(v[(h << C) + j], v[(h << C) + j + HALF], o[(h << C) + j], o[(h << C) + j + HALF]);
+}
+
+// 2^RL adjacent words in 16-byte accesses (the address is a multiple of 16 bytes: limbs are)
+template <int R>
+__device__ __forceinline__ void load_adjacent(const u64* p, u64 (&w)[R]) {
+#pragma unroll
+    for (int j = 0; j < R; j += 2) {
+        const ulonglong2 t = *reinterpret_cast<const ulonglong2*>(p + j);
+        w[j] = t.x; w[j + 1] = t.y;
+    }
+}
+template <int R>
+__device__ __forceinline__ void store_adjacent(u64* p, const u64 (&w)[R]) {
+#pragma unroll
+    for (int j = 0; j < R; j += 2) *reinterpret_cast<ulonglong2*>(p + j) = make_ulonglong2(w[j], w[j + 1]);
+}
+
+// shapes
+template <int SA, int SB, int RL>
+struct FineStrided {          // 16 adjacent columns, all rows
+    static constexpr int CW = 16, LANES = (1 << SA) >> RL, THREADS = CW * LANES, TILES = (1 << SB) / CW, LDS_WORDS = (1 << SA) * CW;
+};
+template <int SA, int SB, int RL>
+struct FineRow {              // rows of 2^SB words, as many as the lanes of a strided tile hold: both passes have the same tile count
+    static constexpr int THREADS = FineStrided<SA, SB, RL>::THREADS, U = (1 << SB) >> RL, ROWS = THREADS / U, TILES = (1 << SA) / ROWS;
+    static_assert(TILES == FineStrided<SA, SB, RL>::TILES, "tile counts");
+    static constexpr int PITCH = (1 << SB) + (1 << SB) / 16, LDS_WORDS = ROWS * PITCH;
+};
+template <int S, int RL>
+struct FineWhole {
+    static constexpr int THREADS = (1 << S) >> RL, LDS_WORDS = (1 << S) + (1 << S) / 16;
+};
+
+}  // namespace ckks

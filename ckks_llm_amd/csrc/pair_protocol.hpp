@@ -22,7 +22,7 @@
 namespace ckks {
 namespace pair {
 
-constexpr unsigned TILES = 16;
+constexpr unsigned TILES = 16;     // at most; a smaller ring's limb has fewer (the template argument T below)
 constexpr unsigned ALL = (1u << TILES) - 1;
 // what the deciding lane tells its workgroup
 constexpr unsigned GO = 16;        // all first-pass tiles are complete: run the second pass of the tiles this workgroup ran
@@ -79,17 +79,18 @@ __host__ __device__ __forceinline__ unsigned claim_own(unsigned* w, unsigned til
 }
 // After a first-pass tile of this workgroup is complete (its stores acknowledged): count it, then decide what comes next -
 // another first-pass tile to run (0..15), GO, or DEFER.
+template <unsigned T = TILES>
 __host__ __device__ __forceinline__ unsigned tile_done_then_decide(unsigned* w, bool stealing, unsigned spin_steal, unsigned spin_max) {
     (void)Atomics::fetch_add(w + DONE, 1u);
     for (;;) {
         for (unsigned n = 0; n <= spin_steal; n++) {
-            if (Atomics::load(w + DONE) == TILES) return GO;
+            if (Atomics::load(w + DONE) == T) return GO;
             Atomics::pause();
         }
         if (stealing) {
-            const unsigned claimed = Atomics::load(w + CLAIM) & ALL;
-            if (claimed != ALL) {
-                const unsigned s = (unsigned)__builtin_ctz(~claimed & ALL);
+            const unsigned claimed = Atomics::load(w + CLAIM) & ((1u << T) - 1u);
+            if (claimed != (1u << T) - 1u) {
+                const unsigned s = (unsigned)__builtin_ctz(~claimed & ((1u << T) - 1u));
                 const unsigned old = Atomics::fetch_or(w + CLAIM, 1u << s);
                 if (!((old >> s) & 1u)) { (void)Atomics::fetch_add(w + STOLEN_TOTAL, 1u); return s; }      // taken over: run it
                 continue;                                    // its own workgroup (or another waiter) was quicker: wait on
@@ -97,7 +98,7 @@ __host__ __device__ __forceinline__ unsigned tile_done_then_decide(unsigned* w, 
         }
         // every tile is in somebody's hands: they are running
         for (unsigned n = 0; n < spin_max; n++) {
-            if (Atomics::load(w + DONE) == TILES) return GO;
+            if (Atomics::load(w + DONE) == T) return GO;
             Atomics::pause();
         }
         return DEFER;

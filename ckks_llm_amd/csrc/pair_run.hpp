@@ -1,0 +1,124 @@
+// Device side of the paired (one-launch) transforms: how a workgroup of the launch asks its limb's protocol words (pair_protocol.hpp),
+// which tile of which limb it takes, and the sequence of its two passes.
+#pragma once
+#include "ntt_core.hpp"
+#include "pair_protocol.hpp"
+
+namespace ckks {
+
+// The two questions that a workgroup of a paired launch asks of its limb's protocol words (pair_protocol.hpp) with atomics that
+// return an answer - the claim of its own first-pass tile and its counting out - ride inside a tile: lane 0 asks behind the
+// tile's own loads (memory operations return in the order of their issue, so an answer that queues behind the other workgroups'
+// atomics on the same words does not hold the loads up) and publishes the answer in LDS, the claim just ahead of the tile's
+// first barrier, the count at the tile's end.  Behind that barrier every lane knows whether a claimed tile is this workgroup's;
+// up to there a tile only reads global memory and writes LDS, so a tile that turns out to be another's leaves no trace.
+// Default: nothing to ask.
+struct TileClaim {
+    unsigned* lds = nullptr;       // where the answer is published (nullptr: nothing to ask)
+    unsigned* words = nullptr;     // the limb's protocol words
+    unsigned tile = 0;
+    bool counting_out = false;     // false: the claim of a first-pass tile; true: the counting out, inside a second-pass tile
+    // start() only issues the atomic and returns what it will bring, untouched: anything computed from it here would make the
+    // wave wait for it at this point; publish() is where it is first looked at
+    __device__ __forceinline__ unsigned start(unsigned tid) const {
+        unsigned v = 0;
+        if (lds && tid == 0) {
+            asm volatile("" ::: "memory");
+            v = counting_out ? pair::Atomics::fetch_add(words + pair::LEFT, 1u) : pair::Atomics::fetch_or(words + pair::CLAIM, 1u << tile);
+        }
+        return v;
+    }
+    // claim: the tile, or LEAVE if it was taken; counting out: how many had left before (the last one out sees TILES - 1)
+    __device__ __forceinline__ void publish(unsigned tid, unsigned raw) const {
+        if (lds && tid == 0) *lds = counting_out ? raw : ((raw >> tile) & 1u ? pair::LEAVE : tile);
+    }
+    __device__ __forceinline__ bool lost() const { return lds && !counting_out && *lds == pair::LEAVE; }
+};
+
+constexpr unsigned PAIR_XCDS = 8;
+constexpr int PAIR_MAX_LIMBS = 4096;               // protocol words per context
+constexpr int PAIR_GROUPED_LIMBS = 40;             // ... and up to this many with a limb's tiles on one XCD, above it spread over all
+constexpr int PAIR_WORD_STRIDE = pair::WORDS;      // protocol words per limb (pair_protocol.hpp)
+constexpr int PAIR_AUTO_LIMBS = 128;               // automatic mode: batches up to this many limbs take the paired kernel (while the grid fits the chip)
+struct PairArgs {
+    unsigned* done;            // [limb * PAIR_WORD_STRIDE] the limb's protocol words (pair_protocol.hpp), zero between launches
+    unsigned* fail;            // host-visible word: nonzero once a wait of the key switch's last launch has run out
+    unsigned limbs;
+    unsigned spin_steal;       // polls after which a waiting workgroup takes over tiles whose workgroups have not started
+    unsigned spin_max;         // polls after which it leaves its second-pass tiles to the last workgroup out
+    unsigned steal;            // 0: no workgroup takes over another's tile (a test setting)
+    unsigned spread;           // the tiles of a limb go to consecutive workgroups, i.e. to all XCDs (larger batches, and a test setting)
+};
+// (limb, tile) of workgroup b of a paired launch
+__device__ __forceinline__ void pair_block(const PairArgs& p, unsigned b, unsigned tiles, unsigned& limb_id, unsigned& tile) {
+    const unsigned idx = b / PAIR_XCDS;
+    limb_id = p.spread ? b / tiles : b % PAIR_XCDS + PAIR_XCDS * (idx / tiles);
+    tile = p.spread ? b % tiles : idx % tiles;
+}
+// The two passes of (limb_id, tile) under the protocol.  pass1(t) and pass2(t) run tile t on the whole workgroup (t is the
+// workgroup's own tile unless it has taken over others; uniform over the workgroup).  stealing = false: a workgroup only ever
+// runs its own tile (the first pass is work that only this workgroup can do, already under way when this is called).
+template <unsigned T = pair::TILES, class P1, class P2>
+__device__ __forceinline__ void pair_run(const PairArgs& p, unsigned limb_id, unsigned tile, unsigned* sh, bool stealing, P1 pass1, P2 pass2) {
+    static_assert(pair::TILES == 16 && T <= pair::TILES, "at most sixteen tiles per limb");
+    unsigned* w = p.done + (size_t)limb_id * PAIR_WORD_STRIDE;
+    // The claim of the own tile travels while the tile's loads do (see TileClaim); a tile taken over later is claimed before it starts.
+    TileClaim own;
+    own.lds = stealing ? sh : nullptr;
+    own.words = w;
+    own.tile = tile;
+    unsigned mine = 0, act = tile;
+    for (bool first = true;; first = false) {
+        pass1(act, first ? own : TileClaim());
+        if (first && own.lost()) { act = pair::LEAVE; break; }                  // uniform: behind the tile's first barrier every lane reads the same word
+        mine |= 1u << act;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_waitcnt(0);                                          // every shared store of this wave has been acknowledged
+        __syncthreads();
+        if (threadIdx.x == 0) *sh = pair::tile_done_then_decide<T>(w, stealing, p.spin_steal, p.spin_max);
+        // The deciding lane's LDS write is complete before its wave reaches the barrier: said explicitly, because a barrier in a
+        // loop has been seen compiled with no wait for a write that reaches it over the loop's back edge.
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        act = *sh;
+        __syncthreads();
+        if (act >= pair::TILES) break;
+    }
+    // Counting out does not wait for the own second pass: nothing that the last workgroup out does (the second pass of tiles that
+    // others have left, the reset of the words) depends on it.  It rides inside the first second-pass tile (see TileClaim); a
+    // workgroup with no second pass to run counts out here.
+    unsigned todo = act == pair::GO ? mine : 0u;
+    TileClaim out;
+    out.lds = sh;
+    out.words = w;
+    out.counting_out = true;
+    if (todo == 0u && threadIdx.x == 0) {
+        if (act == pair::DEFER) pair::defer(w, mine);
+        *sh = pair::Atomics::fetch_add(w + pair::LEFT, 1u);
+    }
+    for (bool first = true; todo; first = false) {
+        const unsigned t = (unsigned)__builtin_ctz(todo);
+        todo &= todo - 1u;
+        __syncthreads();                                                        // the tile before is done with the LDS
+        pass2(t, first ? out : TileClaim());
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);                                         // lgkmcnt(0) only: the LDS write above, not the tile's last stores
+    __syncthreads();
+    if (*sh + 1u != T) return;                                        // how many had counted out before this workgroup
+    // last out: every first-pass tile of the limb is complete; what the others left undone, then the words back to zero
+    __syncthreads();
+    if (threadIdx.x == 0) *sh = pair::Atomics::load(w + pair::TODO) & ((1u << T) - 1u);
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    __syncthreads();
+    const unsigned finished = *sh;
+    todo = finished;
+    while (todo) {
+        const unsigned t = (unsigned)__builtin_ctz(todo);
+        todo &= todo - 1u;
+        __syncthreads();
+        pass2(t, TileClaim());
+    }
+    if (threadIdx.x == 0) pair::reset(w, finished);
+}
+
+}  // namespace ckks

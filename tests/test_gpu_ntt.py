@@ -140,6 +140,38 @@ def test_pseudo_mersenne_backend_at_its_range_ends(logN):
             buf.free()
 
 
+@pytest.mark.parametrize("logN,form", [(12, 1), (13, 1), (14, 1), (13, 2), (14, 2), (15, 2), (16, 2), (13, 3), (14, 3), (15, 3), (16, 3)])
+def test_eight_values_per_lane_forms_match_oracle(logN, form):
+    """Whole limbs in one workgroup, two passes with eight values per lane and the same paired in one launch, for 36-, 49- and 60-bit
+    primes and the general integers (a 55-bit one), with padding limbs and start indices, in both directions; largest residues
+    among them.  The paired form also with polls that run out at once (the last workgroup out then does the second pass), without
+    taking over, and called on two streams of one context in turn."""
+    from ckks_llm_amd.params import small_primes
+    primes = CFG2_Q[:2] + REF_PARAMS[16]["q"][:2] + REF_PARAMS[16]["t"][:2] + small_primes(55, 1 << 17, 1)
+    pair = Pair(logN, [], primes)
+    pair.dev.set_option("ntt_fine", form)
+    N, n = pair.N, len(primes)
+    for polys, first, extra, top in ((1, 0, 0, False), (3, 2, 1, True), (2, 4, 0, False)):
+        mods = n - first
+        plen = mods + 1 + extra
+        data = limbs_uniform(80 + polys, [primes[0]] + primes[first:] + [primes[0]] * extra, polys, N)
+        if top:
+            for j in range(mods):
+                data[:, 1 + j] = primes[first + j] - 1
+        for spin, steal in ((None, True), (0, True), (0, False)) if form == 3 else ((None, True),):
+            pair.dev.set_ntt_chain(0, -1 if spin is None else spin)
+            pair.dev.set_option("pair_no_steal", 0 if steal else 1)
+            for inverse in (False, True):
+                want = data.copy()
+                (pair.orc.FromNTTInplace if inverse else pair.orc.ToNTTInplace)(want.reshape(-1), 1, first, polys, mods, plen)
+                buf = to_dev(data)
+                (pair.dev.FromNTTInplace if inverse else pair.dev.ToNTTInplace)(buf, 1, first, polys, mods, plen)
+                assert np.array_equal(from_dev(buf, data.shape), want), (polys, inverse, spin, steal)
+                buf.free()
+    pair.dev.set_ntt_chain(0, -1)
+    pair.dev.check()
+
+
 def test_n65536_inter_pass_formats():
     """N = 2^16, FP64 back end: primes below 2^39 take the 5-byte inter-pass buffer, 40-bit primes the in-place 8-byte form, and
     ntt_mode 1 forces the in-place form; all against the oracle.  A batch wider than one launch chunk is not needed: chunks
