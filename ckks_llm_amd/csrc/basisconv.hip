@@ -9,6 +9,7 @@
 //     out_k = Barrett( sum_j y_j * ((D/d_j) mod r_k)  -  v * (D mod r_k) ) [ + r_k - sub_k, one conditional subtract ]
 // All of these kernels stream every limb once; they are HBM bound (read nsrc + write ntgt limbs per block).
 #include "context.hpp"
+#include "conv_core.hpp"
 #include "f64_exact.hpp"
 
 namespace ckks {
@@ -150,6 +151,52 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_kernel_split(ConvArgs a, in
     }
 }
 
+// ---- sources and targets below 2^50 or of the form 2^60 - delta (conv_core.hpp): every conversion of the reference's sets ----
+// The targets of a block are shared out over 2^log_parts workgroups, each of which forms the y_j again.  A lane walks through the constants
+// of its targets by scalar loads that follow one another, so a launch that leaves the chip idle is as long as that chain: it is cut
+// until three workgroups per compute unit are there, not further, because scaling eight 60-bit sources costs as much as three
+// targets (N = 2^15, 3 blocks x 2 polynomials of 7 sources: uncut 10.6 us, one target per workgroup 12.9; 2 blocks of 4 sources: 5.6 us in
+// two parts, 6.0 in eight).  On the reference's set at N = 2^16, level 27: 28 limbs to 56 in 17.5 us (128-bit sums: 33), 128 limbs to 64
+// in 37 us (two modular FP64 products per term: 54), which is 2.5 and 2.7 TB/s: the multiply-adds of the scaling and the columns bound it.
+template <int MAXS, int SRC, int TGT>
+__global__ __launch_bounds__(CONV_THREADS) void conv_columns_kernel(ConvArgs a, const ConvBlock* __restrict__ blocks, const PrimeConst* __restrict__ primes,
+                                                                    int log_parts) {
+    const int blk = blockIdx.y >> log_parts, part = blockIdx.y & ((1 << log_parts) - 1);
+    const ConvBlock& b = blocks[blk];          // not aliased by the stores: its entries stay scalar loads
+    const int per = (b.ntgt + (1 << log_parts) - 1) >> log_parts, k_begin = part * per, k_end = min(b.ntgt, k_begin + per);
+    const long x = (long)blockIdx.x * CONV_THREADS + threadIdx.x;
+    const u64* in = a.in + (long)blockIdx.z * a.in_batch_stride;
+    u64* out = a.out + (long)blockIdx.z * a.out_batch_stride + (long)blk * a.out_block_stride;
+    if (k_begin >= k_end) return;                                             // uniform
+    u64 xin[MAXS], y[MAXS];
+    double yd[MAXS];
+#pragma unroll
+    for (int j = 0; j < MAXS; j++) xin[j] = in[(long)b.src_limb[j] * a.N + x];
+    if (b.ncopy && part == 0) {
+#pragma unroll
+        for (int j = 0; j < MAXS; j++)
+            if (j < b.ncopy) out[(long)b.copy_limb[j] * a.N + x] = xin[j];
+    }
+#pragma unroll
+    for (int j = 0; j < MAXS; j++) xin[j] += b.add_in[j];
+    conv_scale<MAXS, SRC>(xin, b, primes, y, yd);
+    const unsigned v = conv_quotient(yd, b, primes);
+    for (int k = k_begin; k < k_end; k++)
+        out[(long)b.tgt_limb[k] * a.N + x] = conv_target<MAXS, TGT>(y, b, k, v, primes[b.tgt_prime[k]], a.centred != 0);
+}
+template <int SRC, int TGT>
+static void launch_conv_columns(ckks_ctx* c, const ConvArgs& a, dim3 grid, const ConvPlan& plan) {
+    const unsigned wgs = grid.x * grid.y * grid.z, enough = 3u * (unsigned)c->cu_count;
+    int parts = 0;                                              // log2 of their number
+    while ((wgs << parts) < enough && (1 << parts) < plan.max_tgt) parts++;
+    grid.y <<= parts;
+    const dim3 block(CONV_THREADS);
+    if (plan.max_src == 1) hipLaunchKernelGGL((conv_columns_kernel<1, SRC, TGT>), grid, block, 0, c->stream, a, a.blocks, a.primes, parts);
+    else if (plan.max_src == 2) hipLaunchKernelGGL((conv_columns_kernel<2, SRC, TGT>), grid, block, 0, c->stream, a, a.blocks, a.primes, parts);
+    else if (plan.max_src <= 4) hipLaunchKernelGGL((conv_columns_kernel<4, SRC, TGT>), grid, block, 0, c->stream, a, a.blocks, a.primes, parts);
+    else hipLaunchKernelGGL((conv_columns_kernel<8, SRC, TGT>), grid, block, 0, c->stream, a, a.blocks, a.primes, parts);
+}
+
 static int launch_conv(ckks_ctx* c, const ConvPlan& plan, u64* out, const u64* in, int batch, long in_bs, long out_bs,
                        long out_block_stride, int centred, int max_src) {
     if (plan.count == 0 || batch <= 0) return CKKS_OK;
@@ -163,6 +210,14 @@ static int launch_conv(ckks_ctx* c, const ConvPlan& plan, u64* out, const u64* i
         if (max_src <= 4) hipLaunchKernelGGL(conv_kernel_f64<4>, grid, block, 0, c->stream, a);
         else if (max_src <= 8) hipLaunchKernelGGL(conv_kernel_f64<8>, grid, block, 0, c->stream, a);
         else hipLaunchKernelGGL(conv_kernel_f64<CONV_MAX_SRC>, grid, block, 0, c->stream, a);
+        CKKS_HIP_TRY(hipGetLastError());
+        return CKKS_OK;
+    }
+    if (plan.src_kind && plan.tgt_kind && plan.max_src <= 8 && plan.max_tgt > 0 && c->arith_mode == 0 && !c->conv_int) {
+        if (plan.src_kind == CONV_SRC_F64 && plan.tgt_kind == CONV_TGT_PM) launch_conv_columns<CONV_SRC_F64, CONV_TGT_PM>(c, a, grid, plan);
+        else if (plan.src_kind == CONV_SRC_PM && plan.tgt_kind == CONV_TGT_F64) launch_conv_columns<CONV_SRC_PM, CONV_TGT_F64>(c, a, grid, plan);
+        else if (plan.src_kind == CONV_SRC_F64) launch_conv_columns<CONV_SRC_F64, CONV_TGT_F64>(c, a, grid, plan);
+        else launch_conv_columns<CONV_SRC_PM, CONV_TGT_PM>(c, a, grid, plan);
         CKKS_HIP_TRY(hipGetLastError());
         return CKKS_OK;
     }

@@ -55,16 +55,16 @@ static void fill_conv_block(ckks::ConvBlock& b, const std::vector<u64>& pqt, con
     std::vector<u64> sp;
     for (int i : src) sp.push_back(pqt[i]);
     for (int j = 0; j < b.nsrc; j++) {
-        b.src_prime[j] = (short)src[j];
-        b.src_limb[j] = (short)src_limb[j];
+        b.src_prime[j] = src[j];
+        b.src_limb[j] = src_limb[j];
         u64 hat = H::prod_mod(sp, 0, b.nsrc, j, sp[j]);
         b.hatinv[j] = H::invmod(hat, sp[j]);
         b.hatinv_s[j] = H::shoup(b.hatinv[j], sp[j]);
     }
     for (int k = 0; k < b.ntgt; k++) {
         u64 r = pqt[tgt[k]];
-        b.tgt_prime[k] = (short)tgt[k];
-        b.tgt_limb[k] = (short)tgt_limb[k];
+        b.tgt_prime[k] = tgt[k];
+        b.tgt_limb[k] = tgt_limb[k];
         for (int j = 0; j < b.nsrc; j++) b.hat[k][j] = H::prod_mod(sp, 0, b.nsrc, j, r);
         b.dmod[k] = H::prod_mod(sp, 0, b.nsrc, -1, r);
     }
@@ -74,8 +74,8 @@ static void fill_conv_block(ckks::ConvBlock& b, const std::vector<u64>& pqt, con
     for (int i : tgt) if (pqt[i] >= (1ull << 41)) b.f64_ok = 0;
     b.split_ok = 1;
     for (int i : tgt) if (pqt[i] >= (1ull << 50)) b.split_ok = 0;
-    if (b.f64_ok)
-        for (int j = 0; j < b.nsrc; j++) b.hatinv_d[j] = balanced_double(b.hatinv[j], sp[j]);
+    for (int j = 0; j < b.nsrc; j++)
+        if (sp[j] < (1ull << 50)) b.hatinv_d[j] = balanced_double(b.hatinv[j], sp[j]);
     if (b.f64_ok || b.split_ok) {
         for (int k = 0; k < b.ntgt; k++) {
             const u64 r = pqt[tgt[k]];
@@ -175,6 +175,10 @@ extern "C" int ckks_ctx_create(ckks_ctx** out, int logN, const uint64_t* p, int 
         P.w1n = it[1]; P.w1n_s = H::shoup(it[1], m);
         P.qd = (double)m; P.qinv_d = 1.0 / (double)m;
         P.n_inv_d = balanced_double(c->n_inv[i], m); P.w1n_d = balanced_double(it[1], m);
+        P.c32_d = P.c60_d = P.c92_d = 0.0;
+        if (m < (1ull << 50)) {
+            P.c32_d = balanced_double(H::powmod(2, 32, m), m); P.c60_d = balanced_double(H::powmod(2, 60, m), m); P.c92_d = balanced_double(H::powmod(2, 92, m), m);
+        }
         P.f64_ok = c->f64_ok[i]; P.pm_delta = pm_delta(m);
     }
 
@@ -305,7 +309,7 @@ extern "C" int ckks_ctx_create(ckks_ctx** out, int logN, const uint64_t* p, int 
                 ckks::ConvBlock blk;
                 fill_conv_block(blk, pqt, iota(p_num + lo, p_num + hi), iota(lo, hi), tg, tg);
                 blk.ncopy = hi - lo;
-                for (int j = 0; j < hi - lo; j++) { blk.copy_prime[j] = (short)(lo + j); blk.copy_limb[j] = (short)(p_num + lo + j); }
+                for (int j = 0; j < hi - lo; j++) { blk.copy_prime[j] = (lo + j); blk.copy_limb[j] = (p_num + lo + j); }
                 blocks.push_back(blk);
             }
             // the same digits with EVERY prime of [P | Q_l] as a target, target k = prime k (for a prime of the digit itself the
@@ -329,7 +333,23 @@ extern "C" int ckks_ctx_create(ckks_ctx** out, int logN, const uint64_t* p, int 
             for (int b = 0; b < pl.count; b++) pl.f64_ok = pl.f64_ok && blocks[pl.first + b].f64_ok;
             pl.split_ok = pl.count > 0;
             for (int b = 0; b < pl.count; b++) pl.split_ok = pl.split_ok && blocks[pl.first + b].split_ok;
+            auto kind = [&](int prime) { return pqt[prime] < (1ull << 50) ? 1 : pm_delta(pqt[prime]) ? 2 : 0; };
+            pl.src_kind = pl.count > 0 ? kind(blocks[pl.first].src_prime[0]) : 0;
+            pl.tgt_kind = pl.count > 0 && blocks[pl.first].ntgt > 0 ? kind(blocks[pl.first].tgt_prime[0]) : 0;
+            for (int b = 0; b < pl.count; b++) {
+                const ckks::ConvBlock& blk = blocks[pl.first + b];
+                pl.max_src = std::max(pl.max_src, blk.nsrc);
+                for (int j = 0; j < blk.nsrc; j++) if (kind(blk.src_prime[j]) != pl.src_kind) pl.src_kind = 0;
+                for (int k = 0; k < blk.ntgt; k++) if (kind(blk.tgt_prime[k]) != pl.tgt_kind) pl.tgt_kind = 0;
+            }
             for (int b = 0; b < pl.count; b++) pl.max_tgt = std::max(pl.max_tgt, blocks[pl.first + b].ntgt);
+        }
+
+    // sources past a block's own (a level may cut a block short): source 0 once more, scaled to zero
+    for (ckks::ConvBlock& blk : blocks)
+        for (int j = blk.nsrc; j < ckks::CONV_MAX_SRC; j++) {
+            blk.src_prime[j] = blk.src_prime[0]; blk.src_limb[j] = blk.src_limb[0];
+            blk.hatinv[j] = blk.hatinv_s[j] = 0; blk.hatinv_d[j] = 0.0; blk.add_in[j] = 0;
         }
 
     // ---- upload ----

@@ -18,6 +18,7 @@ struct PrimeConst {
     u64 w1n, w1n_s;              // psiinv_table[1] (which already carries N^-1, Utils.cuh:200) and its Shoup word
     double qd, qinv_d;           // (double)q and 1/q for the FP64 back end
     double n_inv_d, w1n_d;       // balanced representatives of n_inv, w1n as doubles
+    double c32_d, c60_d, c92_d;  // balanced representatives of 2^32, 2^60, 2^92 modulo primes below 2^50
     int f64_ok;                  // prime small enough for the FP64 back end
     unsigned pm_delta;           // q = 2^60 - pm_delta (below 2^26): the pseudo-Mersenne back end runs it; 0 for every other prime
 };
@@ -27,14 +28,16 @@ constexpr int CONV_MAX_SRC = 16;
 constexpr int CONV_MAX_TGT = 32;
 struct ConvBlock {
     int nsrc, ntgt;
-    short src_prime[CONV_MAX_SRC], src_limb[CONV_MAX_SRC];
-    short tgt_prime[CONV_MAX_TGT], tgt_limb[CONV_MAX_TGT];
+    // whole words: a uniform 16-bit entry is read through the vector memory pipe, and the wait for it also waits for every data load
+    // requested before it
+    int src_prime[CONV_MAX_SRC], src_limb[CONV_MAX_SRC];   // entries from nsrc on repeat source 0 with hatinv = 0: a source of residue zero
+    int tgt_prime[CONV_MAX_TGT], tgt_limb[CONV_MAX_TGT];
     u64 hatinv[CONV_MAX_SRC], hatinv_s[CONV_MAX_SRC];   // (D/d_j)^-1 mod d_j
     u64 hat[CONV_MAX_TGT][CONV_MAX_SRC];                // (D/d_j) mod r_k
     u64 dmod[CONV_MAX_TGT];                             // D mod r_k
     u64 add_in[CONV_MAX_SRC];                           // added to the input residue before scaling (T -> PQ centring)
     u64 sub_out[CONV_MAX_TGT];                          // subtracted from the output residue (T -> PQ centring)
-    short copy_prime[CONV_MAX_SRC], copy_limb[CONV_MAX_SRC];  // ncopy source limbs passed through unchanged
+    int copy_prime[CONV_MAX_SRC], copy_limb[CONV_MAX_SRC];    // ncopy source limbs passed through unchanged
     int ncopy;
     int f64_ok;                                         // every prime of the block is below 2^41: all FP64 tables below are filled
     int split_ok;                                       // every TARGET prime is below 2^50: hat_d, hat31_d and dmod_d are filled
@@ -48,7 +51,9 @@ struct ConvPlan {          // blocks of one map at one level, contiguous in devi
     int first = 0, count = 0;
     bool f64_ok = false;   // all blocks can take the FP64 kernel
     bool split_ok = false; // all blocks can take the kernel that scales in integers and sums in FP64
-    int max_tgt = 0;       // largest number of targets of a block
+    int src_kind = 0;      // 1: every source prime is below 2^50, 2: every one is 2^60 - delta, 0: neither
+    int tgt_kind = 0;      // the same of the targets
+    int max_src = 0, max_tgt = 0;   // largest number of sources, of targets of a block
 };
 
 }  // namespace ckks

@@ -1,0 +1,98 @@
+// Per-coefficient arithmetic of the exact RNS conversions (BasisConv.cuh:18-58) in carry-free integer columns, for source and
+// target primes below 2^50 or of the form 2^60 - delta:
+//     y_j = (x_j + add_j) (D/d_j)^-1 mod d_j,   v = (int) sum_j (double)y_j / (double)d_j,   out_k = sum_j y_j (D/d_j) - v D  mod r_k
+// A product y_j * ((D/d_j) mod r_k) is four 32 x 32 + 64-bit multiply-adds into three columns of weight 1, 2^30, 2^60 (operands split at
+// bit 30) - on this part they issue at the rate of an FP64 FMA - and the columns are reduced once per output.  The forms it replaces took
+// eleven instructions with two carry chains per product (128-bit sums) or fourteen (two modular FP64 products).
+#pragma once
+#include "ntt_core.hpp"
+
+namespace ckks {
+
+enum { CONV_SRC_F64 = 1, CONV_SRC_PM = 2, CONV_TGT_F64 = 1, CONV_TGT_PM = 2 };      // ConvPlan::src_kind, tgt_kind
+
+// v = (int) sum_j (double)y_j / (double)d_j, the terms added in index order, every operation rounded as the reference's: the quotients are
+// taken as products with 1/d_j first.  For at most 16 terms below 1 the two sums differ by less than 2^-43 (16 products off by 2^-52, twice
+// 16 additions of values below 16 off by 2^-49), so where no integer lies within 2^-40 of the fast sum both have the same integer
+// part; elsewhere (about one coefficient in 2^38) the divisions are carried out.  A division costs a dozen instructions.
+// All loops run over MAXS sources: those that a block does not have are residues of zero.
+template <int MAXS>
+__device__ __forceinline__ unsigned conv_quotient(const double (&y)[MAXS], const ConvBlock& b, const PrimeConst* __restrict__ primes) {
+    double s = 0.0;
+#pragma unroll
+    for (int j = 0; j < MAXS; j++)
+        s = __builtin_fma(y[j], primes[b.src_prime[j]].qinv_d, s);
+    constexpr double TOL = 9.094947017729282e-13;                        // 2^-40
+    double f = __builtin_floor(s + TOL);
+    const double g = __builtin_floor(s - TOL);
+    if (f != g && f != 0.0) {
+        double e = 0.0;
+#pragma unroll
+        for (int j = 0; j < MAXS; j++) e += y[j] / primes[b.src_prime[j]].qd;
+        f = (double)(int)e;
+    }
+    return (unsigned)(int)f;
+}
+
+// scaled source residues: as integers and as the doubles that v is formed from
+template <int MAXS, int SRC>
+__device__ __forceinline__ void conv_scale(const u64 (&x)[MAXS], const ConvBlock& b, const PrimeConst* __restrict__ primes, u64 (&y)[MAXS],
+                                           double (&yd)[MAXS]) {
+#pragma unroll
+    for (int j = 0; j < MAXS; j++) {
+        const PrimeConst& ps = primes[b.src_prime[j]];
+        if constexpr (SRC == CONV_SRC_F64) {
+            // x below 2 d (a centring term may have been added), |hatinv| <= d/2: the product lies within 0.9 d of zero
+            yd[j] = canon_f64(mulmod_f64(exact_u2d(x[j]), b.hatinv_d[j], ps.qd, ps.qinv_d), ps.qd, ps.qinv_d);
+            y[j] = bits52(yd[j]);
+        } else {
+            const PmArith ar(ps);
+            y[j] = ar.canonical(ar.mulmod(x[j], b.hatinv[j] << 4));
+            yd[j] = (double)y[j];
+        }
+    }
+}
+
+// columns of one output; at most 8 sources (the middle column then holds 16 products below 2^60 and one of v)
+template <int MAXS>
+__device__ __forceinline__ PmSum conv_columns(const u64 (&y)[MAXS], const u64* __restrict__ hat, unsigned v, u64 neg_dmod) {
+    static_assert(MAXS <= 8, "columns of at most eight products");
+    constexpr unsigned M30 = PmSum::MASK30;
+    PmSum s;
+    s.a0 = (u64)v * ((unsigned)neg_dmod & M30);
+    s.a1 = (u64)v * (unsigned)(neg_dmod >> 30);
+#pragma unroll
+    for (int j = 0; j < MAXS; j++) s.add(y[j], hat[j]);
+    return s;
+}
+// columns of products of words below 2^60 with words below 2^50 -> residue modulo a prime below 2^50: with lo = a0 + (a1 mod 2^30) 2^30 below
+// 2^63.3 and hi = a2 + a1 / 2^30 below 2^54 the sum is lo + hi 2^60; its four halves of at most 32 bits are exact doubles, every modular
+// product lies within 0.51 q of zero.
+__device__ __forceinline__ double conv_reduce_f64(const PmSum& s, const PrimeConst& p) {
+    const u64 lo = s.a0 + ((u64)((unsigned)s.a1 & PmSum::MASK30) << 30), hi = s.a2 + (s.a1 >> 30);
+    const double q = p.qd, qi = p.qinv_d;
+    double r = (double)(unsigned)lo + mulmod_f64((double)(unsigned)(lo >> 32), p.c32_d, q, qi);
+    r += mulmod_f64((double)(unsigned)hi, p.c60_d, q, qi) + mulmod_f64((double)(unsigned)(hi >> 32), p.c92_d, q, qi);
+    return canon_f64(r, q, qi);                                          // |r| < 2^32 + 1.6 q
+}
+
+// residue of target k of the block, canonical; sub: subtracted at the end (the centring of T -> PQ), 0 for none
+template <int MAXS, int TGT>
+__device__ __forceinline__ u64 conv_target(const u64 (&y)[MAXS], const ConvBlock& b, int k, unsigned v, const PrimeConst& pr, bool centred) {
+    const PmSum s = conv_columns(y, b.hat[k], v, pr.q - b.dmod[k]);
+    if constexpr (TGT == CONV_TGT_PM) {
+        const PmArith ar(pr);
+        u64 r = s.reduce(ar);
+        if (centred) r += pr.q - b.sub_out[k];
+        return ar.canonical(r);
+    } else {
+        double r = conv_reduce_f64(s, pr);
+        if (centred) {
+            r -= exact_u2d(b.sub_out[k]);
+            r = r < 0.0 ? r + pr.qd : r;
+        }
+        return bits52(r);
+    }
+}
+
+}  // namespace ckks

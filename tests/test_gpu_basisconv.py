@@ -351,3 +351,47 @@ def test_keyswitch_23_with_more_digits_than_a_carry_free_sum_holds(logN):
             s1, s2, s3 = DeviceBuffer(8 * N * T * QB), DeviceBuffer(8 * N * T * RB * 2), DeviceBuffer(8 * N * T * RB * 2)
             d.keyswitch_23(do, to_dev(d2), dswk, l, s1, s2, s3)
             assert np.array_equal(from_dev(do, wout.shape)[:, :l + 1], wout[:, :l + 1]), (largest, l)
+
+
+@pytest.mark.parametrize("params,logN", [(13, 8), (14, 8), (15, 9), (16, 8)])
+def test_conversions_at_the_edges_of_their_quotient(params, logN):
+    """Values within a few units of zero and of the modulus of a block (of -T/2 for the centred T -> PQ): the sum of y_j / d_j then lies
+    within rounding of an integer, where its integer part is taken from the divisions themselves.  And the largest residues everywhere."""
+    pair = ref_pair(params, logN)
+    o, d, N = pair.orc, pair.dev, pair.N
+    K, Q, T, RB, QB, L = o.p_num, o.q_num, o.t_num, o.Ri_blockNum, o.Qj_blockNum, o.L
+    pq, gamma = o.p + o.q, REF_PARAMS[params]["gamma"]
+    edges = [0, 1, 2, 3, 1000, 1 << 40, -1, -2, -3, -1000, -(1 << 40)]
+
+    def limbs(primes, first, groups):
+        """[groups][len(primes)][N]: uniform residues, the values `first + edge` in the first columns, the largest residues in the next."""
+        a = limbs_uniform(500 + params, primes, groups, N)
+        for j, m in enumerate(primes):
+            for i, e in enumerate(edges):
+                a[:, j, i] = (first + e) % m
+            a[:, j, len(edges)] = m - 1
+        return a
+
+    inp = limbs(pq, 0, 1)
+    want = np.zeros((1, RB * T, N), dtype=np.uint64)
+    o.modUpPQtoT_23(want.reshape(-1), inp.reshape(-1), L, 1)
+    dout = to_dev(np.zeros_like(want))
+    d.modUpPQtoT_23(dout, to_dev(inp), L, 1)
+    assert np.array_equal(from_dev(dout, want.shape), want)
+    for l in (L, 0):
+        inq = limbs(o.q, 0, 1)
+        want = np.zeros((1, QB * T, N), dtype=np.uint64)
+        o.modUpQjtoT_23(want.reshape(-1), inq.reshape(-1), l, 1)
+        dout = to_dev(np.zeros_like(want))
+        d.modUpQjtoT_23(dout, to_dev(inq), l, 1)
+        assert np.array_equal(from_dev(dout, want.shape), want), l
+    half = 1
+    for m in o.t:
+        half *= m
+    half //= 2
+    tt = limbs(o.t, -half, RB).reshape(1, RB * T, N)
+    want = np.zeros((1, RB * T, N), dtype=np.uint64)
+    o.modUpTtoPQl_23(want.reshape(-1), tt.reshape(-1), L, 1)
+    dout = to_dev(np.zeros_like(want))
+    d.modUpTtoPQl_23(dout, to_dev(tt), L, 1)
+    assert np.array_equal(from_dev(dout, want.shape)[:, :K + L + 1], want[:, :K + L + 1])
