@@ -404,6 +404,17 @@ __global__ __launch_bounds__(CONV_THREADS) void rescale_kernel(u64* a, const u64
 
 static bool level_ok(const ckks_ctx* c, int l) { return c && l >= 0 && l <= c->L; }
 
+// the maps with strides of the caller's (words between the polynomials of a batch)
+int launch_modup_t_to_pql(ckks_ctx* c, uint64_t* out, const uint64_t* in, int l, int batch, long in_stride, long out_stride) {
+    return launch_conv(c, c->plan_t_to_pq[l], (u64*)out, (const u64*)in, batch, in_stride, out_stride, 0, 1, c->t_num);
+}
+int launch_modup_qj_to_t(ckks_ctx* c, uint64_t* out, const uint64_t* in, int l, int batch, long in_stride, long out_stride) {
+    return launch_conv(c, c->plan_qj_to_t[l], (u64*)out, (const u64*)in, batch, in_stride, out_stride, 0, 0, c->p_num);
+}
+int launch_moddown_pql_to_ql(ckks_ctx* c, uint64_t* out, const uint64_t* in, int l, int batch, long in_stride, long out_stride) {
+    return launch_moddown(c, (u64*)out, (const u64*)in, l, batch, in_stride, out_stride);
+}
+
 }  // namespace ckks
 
 using namespace ckks;

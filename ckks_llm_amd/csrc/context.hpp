@@ -177,6 +177,11 @@ int launch_hybrid_front_fused(ckks_ctx* c, const uint64_t* in_ntt, uint64_t* wor
 // modulo each remaining prime, its forward transform and the final subtraction and scaling in two launches; *done = false where
 // it does not apply.
 int launch_rescale_fused(ckks_ctx* c, uint64_t* cipher, int l, const uint64_t* inv, bool* done);
+// The maps modUpTtoPQl_23, modUpQjtoT_23 and modDownPQltoQl_23 on `batch` polynomials with strides of the caller's, in words.  The ModDown may
+// write over its own Q limbs (out = in + p_num limbs): a coefficient's output only depends on words that no other output overwrites.
+int launch_modup_t_to_pql(ckks_ctx* c, uint64_t* out, const uint64_t* in, int l, int batch, long in_stride, long out_stride);
+int launch_modup_qj_to_t(ckks_ctx* c, uint64_t* out, const uint64_t* in, int l, int batch, long in_stride, long out_stride);
+int launch_moddown_pql_to_ql(ckks_ctx* c, uint64_t* out, const uint64_t* in, int l, int batch, long in_stride, long out_stride);
 // End of a key switch (ModDown of two extended polynomials, forward transform of the results) with the ModDown inside the first
 // pass of the transform; *done = false where it does not apply (the caller then runs the separate steps).  With addend set, limb
 // i of result z leaves as its sum with addend[(z * addend_poly_stride + i) * N ...] (NTT domain, canonical).

@@ -14,6 +14,7 @@
 #include <string>
 
 #include "context.hpp"
+#include "ntt_core.hpp"
 
 using namespace ckks;
 
@@ -58,26 +59,64 @@ __device__ __forceinline__ u128w fold60(const Sum60& s, u64 extra) {       // s0
     r.lo = lo;
     return r;
 }
-// FAST: every T prime below 2^60 and at most 16 digits (so at most 16 terms per sum): the carry-free sums above
-template <bool FAST>
+// The sums of a rotation and of a baby step in three forms: MODE 2 every T prime is 2^60 - delta (three carry-free columns and a reduction
+// of a dozen instructions), MODE 1 every T prime is below 2^60 and there are at most 16 digits (four columns, one Barrett reduction), MODE 0
+// 128-bit sums.  value(extra): sum + extra mod q, canonical except in MODE 2, where it is below 2^60 + 2^30.
+template <int MODE>
 struct Acc;
 template <>
-struct Acc<true> {
-    Sum60 s{0, 0, 0, 0};
-    __device__ __forceinline__ void mac(u64 a, u64 b) { mac60(s, a, b); }
-    __device__ __forceinline__ u128w value(u64 extra) const { return fold60(s, extra); }
+struct Acc<2> {
+    PmSum s;
+    __device__ __forceinline__ void mac(u64 a, u64 b) { s.add(a, b); }
+    __device__ __forceinline__ void eight(const PrimeConst& p) { s.renormalise(PmArith(p)); }
+    __device__ __forceinline__ u64 value(u64 extra, const PrimeConst& p) const { const PmArith ar(p); return ar.fold(s.reduce(ar) + extra); }
+    static __device__ __forceinline__ u64 canonical(u64 x, const PrimeConst& p) { return PmArith(p).canonical(x); }
 };
 template <>
-struct Acc<false> {
+struct Acc<1> {
+    Sum60 s{0, 0, 0, 0};
+    __device__ __forceinline__ void mac(u64 a, u64 b) { mac60(s, a, b); }
+    __device__ __forceinline__ void eight(const PrimeConst&) {}
+    __device__ __forceinline__ u64 value(u64 extra, const PrimeConst& p) const { return barrett128(fold60(s, extra), p.q, p.mu_hi, p.mu_lo); }
+    static __device__ __forceinline__ u64 canonical(u64 x, const PrimeConst&) { return x; }
+};
+template <>
+struct Acc<0> {
     u128w s{0, 0};
     __device__ __forceinline__ void mac(u64 a, u64 b) { mac128(s, a, b); }
-    __device__ __forceinline__ u128w value(u64 extra) const {
+    __device__ __forceinline__ void eight(const PrimeConst&) {}
+    __device__ __forceinline__ u64 value(u64 extra, const PrimeConst& p) const {
         u128w r = s;
         r.lo += extra;
         r.hi += (r.lo < extra);
-        return r;
+        return barrett128(r, p.q, p.mu_hi, p.mu_lo);
     }
+    static __device__ __forceinline__ u64 canonical(u64 x, const PrimeConst&) { return x; }
 };
+// <digits, key> of one slot, both halves of the key.  Four digits' words are requested together (places past the last digit read the last
+// one again and count as zero): with one digit at a time the lane waited for memory once per digit.
+template <int MODE>
+__device__ __forceinline__ void digit_sums(Acc<MODE>& s1, Acc<MODE>& s2, const u64* up, const u64* key, size_t up_step, size_t key_step, size_t key_half,
+                                           int digits, const PrimeConst& p) {
+    constexpr int H = 4;
+    for (int i0 = 0; i0 < digits; i0 += H) {
+        u64 d[H], k1[H], k2[H];
+#pragma unroll
+        for (int i = 0; i < H; i++) {
+            const int at = i0 + i < digits ? i0 + i : digits - 1;
+            d[i] = up[(size_t)at * up_step];
+            k1[i] = key[(size_t)at * key_step];
+            k2[i] = key[(size_t)at * key_step + key_half];
+        }
+#pragma unroll
+        for (int i = 0; i < H; i++) {
+            const u64 x = i0 + i < digits ? d[i] : 0;
+            s1.mac(x, k1[i]);
+            s2.mac(x, k2[i]);
+        }
+        if (i0 & H) { s1.eight(p); s2.eight(p); }
+    }
+}
 
 // Workgroup id -> (256-slot chunk, T prime, block).  The digits of a, P b and the plaintexts of a (chunk, prime) are the same for
 // every block; workgroups whose ids agree modulo 8 share an XCD and its L2 and start in id order, so the blocks of one (chunk,
@@ -117,68 +156,70 @@ struct GiantArgs {
 
 // one lane per (block, T prime, slot); per rotation of the giant step the rotated pair is formed once and multiplied into the
 // accumulators of all baby steps
-template <int BS, bool FAST>
+template <int BS, int MODE>
 __global__ __launch_bounds__(THREADS) void giant_rotate_mult_kernel(GiantArgs a) {
     const TileIndex ti = tile_index(blockIdx.x, (int)(a.N / THREADS), a.T, a.blocks);
     const long x = (long)ti.chunk * THREADS + threadIdx.x;
     const int k = ti.k, blk = ti.blk;
-    const PrimeConst p = a.primes[a.prime0 + k];
+    const PrimeConst& p = a.primes[a.prime0 + k];
     const long N = a.N;
     const u64 mask = 2 * (u64)N - 1;
     const size_t half = (size_t)a.RB * a.T * N;
     const size_t limb = ((size_t)blk * a.T + k) * N;
-    Acc<false> acc_a[BS], acc_b[BS];         // 128-bit sums here: the carry-free form would double their registers
+    Acc<MODE == 2 ? 2 : 0> acc_a[BS], acc_b[BS];         // 128-bit sums where four columns per sum would double their registers
     for (int j = 0; j < a.gs; j++) {
         const u64* key = a.key[j];
-        u64 ea, eb;
+        u64 ea, eb, mx[BS];
+#pragma unroll
+        for (int i = 0; i < BS; i++)
+            if (i < a.bs && j < a.acc_num[i]) mx[i] = a.plain[i * a.gs + j][(size_t)k * N + x];
         if (!key) {
             ea = a.pqT[limb + x];
             eb = a.pqT[limb + x + half];
         } else {
             const long px = hoist_perm(a.pow[j], x, a.logN, mask);
-            Acc<FAST> s1, s2;
-            for (int i = 0; i < a.digits; i++) {
-                const u64 d = a.up[((size_t)i * a.T + k) * N + px];
-                const size_t kidx = ((size_t)i * a.T * a.RB + (size_t)blk * a.T + k) * N + px;
-                s1.mac(d, key[kidx]);
-                s2.mac(d, key[half * a.dnum + kidx]);
-            }
+            Acc<MODE> s1, s2;
             const u64 b0 = a.pqT[limb + px + half];
-            ea = barrett128(s1.value(0), p.q, p.mu_hi, p.mu_lo);
-            eb = barrett128(s2.value(b0), p.q, p.mu_hi, p.mu_lo);
+            digit_sums<MODE>(s1, s2, a.up + (size_t)k * N + px, key + limb + px, (size_t)a.T * N, half, half * a.dnum, a.digits, p);
+            ea = s1.value(0, p);
+            eb = s2.value(b0, p);
         }
 #pragma unroll
         for (int i = 0; i < BS; i++)
             if (i < a.bs && j < a.acc_num[i]) {
-                const u64 mx = a.plain[i * a.gs + j][(size_t)k * N + x];
-                acc_a[i].mac(ea, mx);
-                acc_b[i].mac(eb, mx);
+                acc_a[i].mac(ea, mx[i]);
+                acc_b[i].mac(eb, mx[i]);
             }
+        if ((j & 7) == 7) {
+#pragma unroll
+            for (int i = 0; i < BS; i++) { acc_a[i].eight(p); acc_b[i].eight(p); }
+        }
     }
 #pragma unroll
     for (int i = 0; i < BS; i++)
         if (i < a.bs) {
-            a.out[limb + x + (size_t)(2 * i) * half] = barrett128(acc_a[i].value(0), p.q, p.mu_hi, p.mu_lo);
-            a.out[limb + x + (size_t)(2 * i + 1) * half] = barrett128(acc_b[i].value(0), p.q, p.mu_hi, p.mu_lo);
+            a.out[limb + x + (size_t)(2 * i) * half] = acc_a[i].canonical(acc_a[i].value(0, p), p);
+            a.out[limb + x + (size_t)(2 * i + 1) * half] = acc_b[i].canonical(acc_b[i].value(0, p), p);
         }
 }
 
 struct BabyArgs {
     u64* out;                       // [a | b][Ri_blockNum][t_num], accumulated in place
-    const u64* up;
-    const u64* in;                  // the pair that is rotated; only its b half is read
+    const u64* up;                  // digits of rotation r at up + r * up_stride
+    const u64* in;                  // the pair that rotation r rotates, at in + r * in_stride; only its b half is read
     const PrimeConst* primes;
     const u64* key[MAX_GS];
     u64 pow[MAX_GS];
     long N;
+    size_t up_stride, in_stride;    // words; zero when every rotation is of the same pair
     int logN, T, RB, dnum, digits, prime0, rot_num, blocks;
 };
-template <bool FAST>
+template <int MODE>
 __global__ __launch_bounds__(THREADS) void baby_rotate_kernel(BabyArgs a) {
     const TileIndex ti = tile_index(blockIdx.x, (int)(a.N / THREADS), a.T, a.blocks);
     const long x = (long)ti.chunk * THREADS + threadIdx.x;
     const int k = ti.k, blk = ti.blk;
-    const PrimeConst p = a.primes[a.prime0 + k];
+    const PrimeConst& p = a.primes[a.prime0 + k];
     const long N = a.N;
     const u64 mask = 2 * (u64)N - 1;
     const size_t half = (size_t)a.RB * a.T * N;
@@ -190,23 +231,15 @@ __global__ __launch_bounds__(THREADS) void baby_rotate_kernel(BabyArgs a) {
         if (!key) continue;
         any = true;
         const long px = hoist_perm(a.pow[r], x, a.logN, mask);
-        Acc<FAST> s1, s2;
-        for (int i = 0; i < a.digits; i++) {
-            const u64 d = a.up[((size_t)i * a.T + k) * N + px];
-            const size_t kidx = ((size_t)i * a.T * a.RB + (size_t)blk * a.T + k) * N + px;
-            s1.mac(d, key[kidx]);
-            s2.mac(d, key[half * a.dnum + kidx]);
-        }
-        const u64 b0 = a.in[limb + px + half];
-        u128w v1 = s1.value(oa), v2 = s2.value(b0);
-        v2.lo += ob;
-        v2.hi += (v2.lo < ob);
-        oa = barrett128(v1, p.q, p.mu_hi, p.mu_lo);
-        ob = barrett128(v2, p.q, p.mu_hi, p.mu_lo);
+        Acc<MODE> s1, s2;
+        const u64 b0 = a.in[r * a.in_stride + limb + px + half];
+        digit_sums<MODE>(s1, s2, a.up + r * a.up_stride + (size_t)k * N + px, key + limb + px, (size_t)a.T * N, half, half * a.dnum, a.digits, p);
+        oa = s1.value(oa, p);
+        ob = s2.value(b0 + ob, p);                      // two residues below 2^62: no carry
     }
     if (any) {
-        a.out[limb + x] = oa;
-        a.out[limb + x + half] = ob;
+        a.out[limb + x] = Acc<MODE>::canonical(oa, p);
+        a.out[limb + x + half] = Acc<MODE>::canonical(ob, p);
     }
 }
 
@@ -248,12 +281,31 @@ __global__ __launch_bounds__(THREADS) void rescale_coeff_kernel(u64* a, const Pr
     a[idx] = mul_shoup(ra, inv[i], inv_s[i], q);
 }
 
-// the carry-free sums need every operand below 2^60 and at most 16 terms per sum
-bool carry_free_ok(const ckks_ctx* c, int digits) {
-    if (digits > 16 || c->arith_mode == 1) return false;
-    for (int k = 0; k < c->t_num; k++)
-        if (c->pqt[(size_t)c->p_num + c->q_num + k] >= (1ull << 60)) return false;
-    return true;
+// which form the sums take: the four columns need every operand below 2^60 and at most 16 terms per sum
+int sum_mode(const ckks_ctx* c, int digits) {
+    if (c->arith_mode == 1) return 0;
+    bool pm = true, below = digits <= 16;
+    for (int k = 0; k < c->t_num; k++) {
+        pm = pm && ntt_back_end(c, c->p_num + c->q_num + k) == 3;
+        below = below && c->pqt[(size_t)c->p_num + c->q_num + k] < (1ull << 60);
+    }
+    return pm ? 2 : below ? 1 : 0;
+}
+template <int MODE>
+void launch_giant(ckks_ctx* c, dim3 grid, const GiantArgs& a) {
+    const dim3 block(THREADS);
+    if (a.bs == 1) hipLaunchKernelGGL((giant_rotate_mult_kernel<1, MODE>), grid, block, 0, c->stream, a);
+    else if (a.bs == 2) hipLaunchKernelGGL((giant_rotate_mult_kernel<2, MODE>), grid, block, 0, c->stream, a);
+    else if (a.bs <= 4) hipLaunchKernelGGL((giant_rotate_mult_kernel<4, MODE>), grid, block, 0, c->stream, a);
+    else hipLaunchKernelGGL((giant_rotate_mult_kernel<8, MODE>), grid, block, 0, c->stream, a);
+}
+void launch_baby(ckks_ctx* c, const BabyArgs& a) {
+    const dim3 grid((unsigned)(c->N / THREADS) * (unsigned)c->t_num * (unsigned)a.blocks), block(THREADS);
+    switch (sum_mode(c, a.digits)) {
+        case 2: hipLaunchKernelGGL(baby_rotate_kernel<2>, grid, block, 0, c->stream, a); break;
+        case 1: hipLaunchKernelGGL(baby_rotate_kernel<1>, grid, block, 0, c->stream, a); break;
+        default: hipLaunchKernelGGL(baby_rotate_kernel<0>, grid, block, 0, c->stream, a);
+    }
 }
 
 int need_t_basis(const ckks_ctx* c, int l, const char* who) {
@@ -328,19 +380,33 @@ extern "C" int ckks_giant_rotate_mult_plain_t(ckks_ctx* c, uint64_t* bs_cipher_T
         }
     const int blockNum = (c->p_num + l + 1 + c->gamma - 1) / c->gamma;
     a.blocks = blockNum;
-    const dim3 grid((unsigned)(c->N / THREADS) * (unsigned)c->t_num * (unsigned)blockNum), block(THREADS);
-    if (carry_free_ok(c, a.digits)) {
-        if (bs == 1) hipLaunchKernelGGL((giant_rotate_mult_kernel<1, true>), grid, block, 0, c->stream, a);
-        else if (bs == 2) hipLaunchKernelGGL((giant_rotate_mult_kernel<2, true>), grid, block, 0, c->stream, a);
-        else if (bs <= 4) hipLaunchKernelGGL((giant_rotate_mult_kernel<4, true>), grid, block, 0, c->stream, a);
-        else hipLaunchKernelGGL((giant_rotate_mult_kernel<8, true>), grid, block, 0, c->stream, a);
-    } else {
-        if (bs == 1) hipLaunchKernelGGL((giant_rotate_mult_kernel<1, false>), grid, block, 0, c->stream, a);
-        else if (bs == 2) hipLaunchKernelGGL((giant_rotate_mult_kernel<2, false>), grid, block, 0, c->stream, a);
-        else if (bs <= 4) hipLaunchKernelGGL((giant_rotate_mult_kernel<4, false>), grid, block, 0, c->stream, a);
-        else hipLaunchKernelGGL((giant_rotate_mult_kernel<8, false>), grid, block, 0, c->stream, a);
+    const dim3 grid((unsigned)(c->N / THREADS) * (unsigned)c->t_num * (unsigned)blockNum);
+    switch (sum_mode(c, a.digits)) {
+        case 2: launch_giant<2>(c, grid, a); break;
+        case 1: launch_giant<1>(c, grid, a); break;
+        default: launch_giant<0>(c, grid, a);
     }
     CKKS_HIP_TRY(hipGetLastError());
+    return CKKS_OK;
+}
+
+// the arguments of a launch of baby_rotate_kernel on one pair
+static int baby_args(ckks_ctx* c, BabyArgs& a, uint64_t* output, const uint64_t* modUp_QjtoT, const uint64_t* input, int rotNum,
+                     const uint64_t* const* rotKeys_host, const int* rotSlots_host, int l) {
+    a.out = (u64*)output; a.up = (const u64*)modUp_QjtoT; a.in = (const u64*)input; a.primes = c->d_primes;
+    a.N = c->N; a.logN = c->logN; a.T = c->t_num; a.RB = c->Ri_blockNum; a.dnum = c->dnum;
+    a.digits = (l + 1 + c->p_num - 1) / c->p_num; a.prime0 = c->p_num + c->q_num; a.rot_num = rotNum; a.up_stride = a.in_stride = 0;
+    if (a.digits > c->dnum) { set_error("hoisted rotations: the level needs more digits than the keys hold (q_num is no multiple of p_num)"); return CKKS_E_INVALID; }
+    for (int r = 0; r < MAX_GS; r++) {
+        a.key[r] = r < rotNum ? (const u64*)rotKeys_host[r] : nullptr;
+        a.pow[r] = 1;
+        if (a.key[r]) {
+            if (rotSlots_host[r] < 0) { set_error("Baby_Rotate: a key without its rotation"); return CKKS_E_INVALID; }
+            int rc = ckks_rot_group(c, rotSlots_host[r], &a.pow[r]);
+            if (rc) return rc;
+        }
+    }
+    a.blocks = (c->p_num + l + 1 + c->gamma - 1) / c->gamma;
     return CKKS_OK;
 }
 
@@ -352,26 +418,11 @@ extern "C" int ckks_baby_rotate(ckks_ctx* c, uint64_t* output, const uint64_t* m
     if (rotNum < 0 || rotNum > MAX_GS) { set_error("Baby_Rotate: at most 16 rotations per call"); return CKKS_E_INVALID; }
     if (output == input) { set_error("Baby_Rotate: output and input must be different buffers"); return CKKS_E_INVALID; }
     BabyArgs a;
-    a.out = (u64*)output; a.up = (const u64*)modUp_QjtoT; a.in = (const u64*)input; a.primes = c->d_primes;
-    a.N = c->N; a.logN = c->logN; a.T = c->t_num; a.RB = c->Ri_blockNum; a.dnum = c->dnum;
-    a.digits = (l + 1 + c->p_num - 1) / c->p_num; a.prime0 = c->p_num + c->q_num; a.rot_num = rotNum;
-    if (a.digits > c->dnum) { set_error("hoisted rotations: the level needs more digits than the keys hold (q_num is no multiple of p_num)"); return CKKS_E_INVALID; }
+    if ((rc = baby_args(c, a, output, modUp_QjtoT, input, rotNum, rotKeys_host, rotSlots_host, l))) return rc;
     bool any = false;
-    for (int r = 0; r < MAX_GS; r++) {
-        a.key[r] = r < rotNum ? (const u64*)rotKeys_host[r] : nullptr;
-        a.pow[r] = 1;
-        if (a.key[r]) {
-            if (rotSlots_host[r] < 0) { set_error("Baby_Rotate: a key without its rotation"); return CKKS_E_INVALID; }
-            if ((rc = ckks_rot_group(c, rotSlots_host[r], &a.pow[r]))) return rc;
-            any = true;
-        }
-    }
+    for (int r = 0; r < MAX_GS; r++) any = any || a.key[r];
     if (!any) return CKKS_OK;
-    const int blockNum = (c->p_num + l + 1 + c->gamma - 1) / c->gamma;
-    a.blocks = blockNum;
-    const dim3 grid((unsigned)(c->N / THREADS) * (unsigned)c->t_num * (unsigned)blockNum);
-    if (carry_free_ok(c, a.digits)) hipLaunchKernelGGL(baby_rotate_kernel<true>, grid, dim3(THREADS), 0, c->stream, a);
-    else hipLaunchKernelGGL(baby_rotate_kernel<false>, grid, dim3(THREADS), 0, c->stream, a);
+    launch_baby(c, a);
     CKKS_HIP_TRY(hipGetLastError());
     return CKKS_OK;
 }
@@ -404,9 +455,8 @@ extern "C" int ckks_bsgs_level_23(ckks_ctx* c, uint64_t* cipher, int l, const ui
     uint64_t* up = scratch;
     uint64_t* pq = up + N * T * c->Qj_blockNum;
     uint64_t* pqT = pq + 2 * (size_t)(K + L + 1) * N;
-    uint64_t* gsT = pqT + 2 * half;
-    uint64_t* back = gsT + 2 * half;
-    uint64_t* bsT = back + 2 * half;
+    uint64_t* back = pqT + 2 * half;
+    uint64_t* bsT = back + 4 * half;
     if ((rc = ckks_modup_qj_to_t(c, up, cipher, l, 1))) return rc;                                                  // :262
     if ((rc = launch_ntt(c, up, 0, K + L + 1, cipher_blockNum, T, T, 0, 1, false))) return rc;                      // :263
     if ((rc = ckks_cipher_mul_p(c, pq, cipher, l))) return rc;                                                      // :267
@@ -416,21 +466,34 @@ extern "C" int ckks_bsgs_level_23(ckks_ctx* c, uint64_t* cipher, int l, const ui
     int slots[MAX_GS];
     for (int j = 0; j < gs; j++) { keys[j] = rot_in_host[j] != 0 ? rot_in_keys_host[j] : nullptr; slots[j] = rot_in_host[j] != 0 ? rot_in_host[j] : -1; }
     if ((rc = ckks_giant_rotate_mult_plain_t(c, bsT, pqT, up, keys, slots, plaintextT_host, accNum_host, bs, gs, l))) return rc;   // :308
-    for (int i = 1; i < bs; i++) {                                                                                  // :326-356
-        uint64_t* part = bsT + (size_t)i * 2 * half;
+    // The baby steps (:326-356).  The reference takes one after the other; nothing but the closing sum connects them, so as many as the
+    // scratch in front of bsT holds go through every step together: the a halves (only they are brought down) back to coefficients and
+    // down to [Q], their digits up to T again, and one launch that adds all the rotated pairs, reading the b halves where they are.
+    const size_t per_step = (size_t)(K + L + 1 + cipher_blockNum * T) * N;          // [P | Q_l] limbs, then the digits
+    const size_t fits = (size_t)(bsT - scratch) / per_step;
+    for (int i = 1; i < bs;) {
         if (rot_out_host[i] == 0) {
-            if ((rc = ckks_cipher_add_t(c, bsT, part, RB * 2))) return rc;
+            if ((rc = ckks_cipher_add_t(c, bsT, bsT + (size_t)i * 2 * half, RB * 2))) return rc;
+            i++;
             continue;
         }
-        CKKS_HIP_TRY(hipMemcpyAsync(gsT, part, 2 * half * sizeof(uint64_t), hipMemcpyDeviceToDevice, c->stream));
-        if ((rc = launch_ntt(c, part, 0, K + L + 1, blockNum, T, T, (long)RB * T, 2, true))) return rc;
-        if ((rc = ckks_modup_t_to_pql(c, back, part, l, 1))) return rc;
-        if ((rc = ckks_moddown_pql_to_ql(c, cipher, back, l, 1))) return rc;
-        if ((rc = ckks_modup_qj_to_t(c, up, cipher, l, 1))) return rc;
-        if ((rc = launch_ntt(c, up, 0, K + L + 1, cipher_blockNum, T, T, 0, 1, false))) return rc;
-        const uint64_t* key1[1] = {rot_out_keys_host[i]};
-        const int slot1[1] = {rot_out_host[i]};
-        if ((rc = ckks_baby_rotate(c, bsT, up, gsT, 1, key1, slot1, l))) return rc;
+        int n = 1;
+        while (i + n < bs && rot_out_host[i + n] != 0 && (size_t)n < fits) n++;
+        uint64_t* part = bsT + (size_t)i * 2 * half;
+        uint64_t* low = scratch;                                                    // step s: [P | Q_l] at low + s (K+L+1) N, its Q limbs replaced by the ModDown's
+        uint64_t* dig = scratch + (size_t)n * (K + L + 1) * N;                      // step s: digits at dig + s cipher_blockNum T N
+        if ((rc = launch_ntt(c, part, 0, K + L + 1, blockNum, T, T, 2l * RB * T, n, true))) return rc;
+        if ((rc = launch_modup_t_to_pql(c, low, part, l, n, 2 * (long)half, (long)(K + L + 1) * (long)N))) return rc;
+        if ((rc = launch_moddown_pql_to_ql(c, low + (size_t)K * N, low, l, n, (long)(K + L + 1) * (long)N, (long)(K + L + 1) * (long)N))) return rc;
+        if ((rc = launch_modup_qj_to_t(c, dig, low + (size_t)K * N, l, n, (long)(K + L + 1) * (long)N, (long)cipher_blockNum * T * (long)N))) return rc;
+        if ((rc = launch_ntt(c, dig, 0, K + L + 1, n * cipher_blockNum, T, T, 0, 1, false))) return rc;
+        BabyArgs a;
+        if ((rc = baby_args(c, a, bsT, dig, part, n, rot_out_keys_host + i, rot_out_host + i, l))) return rc;
+        a.up_stride = (size_t)cipher_blockNum * T * N;
+        a.in_stride = 2 * half;
+        launch_baby(c, a);
+        CKKS_HIP_TRY(hipGetLastError());
+        i += n;
     }
     if ((rc = launch_ntt(c, bsT, 0, K + L + 1, blockNum, T, T, (long)RB * T, 2, true))) return rc;                  // :359
     if ((rc = ckks_modup_t_to_pql(c, back, bsT, l, 2))) return rc;                                                  // :361
