@@ -479,6 +479,8 @@ extern "C" int ckks_rescale(ckks_ctx* c, uint64_t* cipher, uint64_t* scratch, in
     bool fused = false;
     if ((rc = launch_rescale_fused(c, cipher, l, inv_l, &fused))) return rc;
     if (fused) return CKKS_OK;
+    if ((rc = launch_rescale_lines(c, cipher, scratch, l, inv_l, &fused))) return rc;
+    if (fused) return CKKS_OK;
     dim3 grid((unsigned)(c->N / CONV_THREADS), l, 2), block(CONV_THREADS);
     hipLaunchKernelGGL(mod_to_qi_kernel, grid, block, 0, c->stream, (u64*)scratch, (const u64*)cipher, c->d_primes, c->N, K, L + 1, l);
     rc = launch_ntt(c, scratch, 0, K, 2, l, L + 1, 0, 1, false);                                   // :376
@@ -501,6 +503,11 @@ int ckks::keyswitch_23_add(ckks_ctx* c, uint64_t* out, uint64_t* d2, const uint6
     const int K = c->K, L = c->L, T = c->t_num, RB = c->Ri_blockNum;
     const int swk_blockNum = (K + l + 1 + c->gamma - 1) / c->gamma, cipher_blockNum = (l + 1 + K - 1) / K;
     int rc;
+    if (!addend) {
+        bool lines = false;
+        if ((rc = launch_keyswitch_lines(c, out, d2, swk, l, up, ext, &lines))) return rc;
+        if (lines) return CKKS_OK;
+    }
     if ((rc = launch_ntt(c, d2, 0, K, 1, l + 1, L + 1, 0, 1, true))) return rc;                     // :219
     if ((rc = ckks_modup_qj_to_t(c, up, d2, l, 1))) return rc;                                      // :221
     if ((rc = launch_ntt(c, up, 0, K + L + 1, cipher_blockNum, T, T, 0, 1, false))) return rc;      // :223

@@ -386,6 +386,36 @@ extern "C" int ckks_ctx_create(ckks_ctx** out, int logN, const uint64_t* p, int 
         }
         up(upload(&c->d_primes_modup, pu));
     }
+    {
+        bool fits = t_num > 0 && t_num <= 8 && gamma > 0 && K > 0 && K <= 8;
+        for (int i = 0; i < PQ && fits; i++) fits = pqt[i] < (1ull << 50);
+        for (int j = 0; j < t_num && fits; j++) fits = pm_delta(tV[j]) != 0;
+        if (fits) {
+            std::vector<ckks::KsDownTarget> tg(PQ);
+            std::vector<ckks::KsDownSource> sr(8);
+            for (int i = 0; i < PQ; i++) {
+                ckks::KsDownTarget& g = tg[i];
+                std::memset(&g, 0, sizeof(g));
+                for (int j = 0; j < t_num; j++) g.hat[j] = c->THatModRi[(size_t)i * t_num + j];
+                g.q = pqt[i]; g.neg_dmod = pqt[i] - c->Tmodpqi[i];
+                g.qd = pc[i].qd; g.qinv = pc[i].qinv_d; g.c32 = pc[i].c32_d; g.c60 = pc[i].c60_d; g.c92 = pc[i].c92_d;
+                g.sub = (double)c->halfTmodpqti[i];
+                if (i < K) g.phat[0] = balanced_double(c->pHatInvVecModp[i], pqt[i]);
+                else {
+                    for (int k = 0; k < K; k++) g.phat[k] = balanced_double(c->pHatVecModq[(size_t)(i - K) * K + k], pqt[i]);
+                    g.pinv = balanced_double(c->PinvModq[i - K], pqt[i]);
+                }
+            }
+            for (int j = 0; j < 8; j++) {
+                const int t = j < t_num ? j : 0;
+                sr[j].hatinv16 = j < t_num ? c->THatInv[j] << 4 : 0;
+                sr[j].add = j < t_num ? c->halfTmodpqti[PQ + j] : 0;
+                sr[j].q = tV[t]; sr[j].qd = pc[PQ + t].qd; sr[j].qinv = pc[PQ + t].qinv_d; sr[j].delta = pm_delta(tV[t]); sr[j].pad = 0;
+            }
+            up(upload(&c->d_down_tgt, tg));
+            up(upload(&c->d_down_src, sr));
+        }
+    }
     up(upload(&c->d_tw_fwd, twf));
     up(upload(&c->d_tw_inv, twi));
     up(upload(&c->d_twd_fwd, twdf));
@@ -420,7 +450,7 @@ extern "C" int ckks_ctx_destroy(ckks_ctx* c) {
     if (!c) return CKKS_OK;
     (void)hipDeviceSynchronize();
     void* ptrs[] = {c->d_primes, c->d_primes_moddown, c->d_primes_modup, c->d_tw_fwd, c->d_tw_inv, c->d_twd_fwd, c->d_twd_inv, c->d_conv, c->d_pHatVecModq,
-                    c->d_pHatInvVecModp, c->d_PinvModq, c->d_qiInvModql, c->d_ntt_chain, c->d_ntt_mid};
+                    c->d_pHatInvVecModp, c->d_PinvModq, c->d_qiInvModql, c->d_ntt_chain, c->d_ntt_mid, c->d_down_tgt, c->d_down_src};
     for (void* p : ptrs) if (p) (void)hipFree(p);
     if (c->d_ntt_pair) (void)hipFree(c->d_ntt_pair);
     if (c->h_pair_fail) (void)hipHostFree(c->h_pair_fail);
@@ -486,7 +516,7 @@ extern "C" int ckks_ctx_set_option(ckks_ctx* c, const char* name, long value) {
     else if (n == "conv_int") c->conv_int = value != 0;
     else if (n == "ntt_no_reverse") c->ntt_no_reverse = value != 0;
     else if (n == "pair_no_steal") c->pair_no_steal = value != 0;
-    else if (n == "ntt_fine") { if (value < 0 || value > 4) return CKKS_E_INVALID; c->ntt_fine = (int)value; }
+    else if (n == "ntt_fine") { if (value < 0 || value > 5) return CKKS_E_INVALID; c->ntt_fine = (int)value; }
     else if (n == "ntt_chunk") { if (value < 0 || value > 65535) return CKKS_E_INVALID; c->ntt_chunk = (int)value; }
     else { ckks::set_error("ckks_ctx_set_option: unknown name " + n); return CKKS_E_INVALID; }
     return CKKS_OK;

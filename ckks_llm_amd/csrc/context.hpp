@@ -47,6 +47,21 @@ struct ConvBlock {
     double dmod_d[CONV_MAX_TGT];
 };
 
+// The constants of T -> [P | Q] and of the ModDown behind it (ks_lines.hip), per prime of [P | Q] and per T prime: whatever a lane needs for one
+// residue in four consecutive cache lines.  They are the same at every level.
+struct KsDownTarget {
+    u64 hat[8];                                         // (T/t_j) mod r
+    u64 q, neg_dmod;                                    // r, r - (T mod r)
+    double qd, qinv, c32, c60, c92, sub;                // sub: the centring constant floor(T/2) mod r
+    double phat[8];                                     // (P/p_i) mod q, balanced; for a special prime phat[0] = (P/p)^-1 mod p
+    double pinv, pad[7];                                // P^-1 mod q, balanced
+};
+struct KsDownSource {
+    u64 hatinv16, add, q;                               // 16 (T/t_j)^-1 mod t_j, floor(T/2) mod t_j
+    double qd, qinv;
+    unsigned delta, pad;
+};
+
 struct ConvPlan {          // blocks of one map at one level, contiguous in device memory
     int first = 0, count = 0;
     bool f64_ok = false;   // all blocks can take the FP64 kernel
@@ -87,6 +102,8 @@ struct ckks_ctx {
     double* d_twd_inv = nullptr;
     ckks::ConvBlock* d_conv = nullptr;    // all conversion blocks
     std::vector<ckks::ConvPlan> plan_pq_to_t, plan_qj_to_t, plan_t_to_pq, plan_hybrid, plan_hybrid_all;   // indexed by level l
+    ckks::KsDownTarget* d_down_tgt = nullptr;   // [K + L + 1], null where the bases are not those of ks_down_kernel
+    ckks::KsDownSource* d_down_src = nullptr;   // [8]: T primes, then sources that count as zero
     // ModDown / rescale constants on device
     uint64_t* d_pHatVecModq = nullptr;    // [L+1][K]
     uint64_t* d_pHatInvVecModp = nullptr; // [K] then [K] Shoup words
@@ -115,7 +132,7 @@ struct ckks_ctx {
     // takes the limbs in forward order; limbs per trip through the inter-pass buffer (0: all)
     bool ks_split = false, ks_back_split = false, conv_int = false, ntt_no_reverse = false, pair_no_steal = false;
     int ntt_chunk = 0;
-    int ntt_fine = 0;                     // 0: small batches take the forms of ntt_fine.hip by the rule there, 1 .. 3: whole limbs / two passes / paired passes wherever they exist, 4: never
+    int ntt_fine = 0;                     // 0: small batches take the forms of ntt_fine.hip by the rule there, 1 .. 3, 5: whole limbs / two passes / paired / paired with half tiles wherever they exist, 4: never
     unsigned* h_pair_fail = nullptr;      // pinned host word that a paired transform raises when one of its waits ran out
     void* d_ntt_chain = nullptr;          // completion words of the chained (one-launch) transform, allocated on its first use; zero between transforms
 };
@@ -177,6 +194,17 @@ int launch_hybrid_front_fused(ckks_ctx* c, const uint64_t* in_ntt, uint64_t* wor
 // modulo each remaining prime, its forward transform and the final subtraction and scaling in two launches; *done = false where
 // it does not apply.
 int launch_rescale_fused(ckks_ctx* c, uint64_t* cipher, int l, const uint64_t* inv, bool* done);
+// Key switch through T, the operations around it and the rescale in five (two) launches at N = 2^12 .. 2^15 (ks_lines.hip); *done = false where
+// they do not apply (nothing launched).  d2: one polynomial of coefficients, tmp: two polynomials, up / ext: the reference's
+// modUp_QjtoT_temp and exProduct_T_temp; pow: exponent of the slot permutation as a scatter.
+int launch_keyswitch_lines(ckks_ctx* c, uint64_t* out, uint64_t* d2, const uint64_t* swk, int l, uint64_t* up, uint64_t* ext, bool* done);
+int launch_mult_lines(ckks_ctx* c, uint64_t* out, const uint64_t* c1, const uint64_t* c2, const uint64_t* swk, int l, uint64_t* d2, uint64_t* up,
+                      uint64_t* ext, bool* done);
+int launch_rotate_lines(ckks_ctx* c, uint64_t* out, const uint64_t* cipher, const uint64_t* key, uint64_t pow, int l, uint64_t* d2, uint64_t* tmp,
+                        uint64_t* up, uint64_t* ext, bool* done);
+int launch_conjugate_lines(ckks_ctx* c, uint64_t* out, const uint64_t* cipher, const uint64_t* key, int l, uint64_t* d2, uint64_t* up, uint64_t* ext,
+                           bool* done);
+int launch_rescale_lines(ckks_ctx* c, uint64_t* cipher, uint64_t* scratch, int l, const uint64_t* inv, bool* done);
 // The maps modUpTtoPQl_23, modUpQjtoT_23 and modDownPQltoQl_23 on `batch` polynomials with strides of the caller's, in words.  The ModDown may
 // write over its own Q limbs (out = in + p_num limbs): a coefficient's output only depends on words that no other output overwrites.
 int launch_modup_t_to_pql(ckks_ctx* c, uint64_t* out, const uint64_t* in, int l, int batch, long in_stride, long out_stride);

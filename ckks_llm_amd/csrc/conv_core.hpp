@@ -16,22 +16,25 @@ enum { CONV_SRC_F64 = 1, CONV_SRC_PM = 2, CONV_TGT_F64 = 1, CONV_TGT_PM = 2 };  
 // 16 additions of values below 16 off by 2^-49), so where no integer lies within 2^-40 of the fast sum both have the same integer
 // part; elsewhere (about one coefficient in 2^38) the divisions are carried out.  A division costs a dozen instructions.
 // All loops run over MAXS sources: those that a block does not have are residues of zero.
+template <class Exact>
+__device__ __forceinline__ unsigned conv_quotient_of(double s, Exact exact) {
+    constexpr double TOL = 9.094947017729282e-13;                        // 2^-40
+    double f = __builtin_floor(s + TOL);
+    const double g = __builtin_floor(s - TOL);
+    if (f != g && f != 0.0) f = (double)(int)exact();
+    return (unsigned)(int)f;
+}
 template <int MAXS>
 __device__ __forceinline__ unsigned conv_quotient(const double (&y)[MAXS], const ConvBlock& b, const PrimeConst* __restrict__ primes) {
     double s = 0.0;
 #pragma unroll
-    for (int j = 0; j < MAXS; j++)
-        s = __builtin_fma(y[j], primes[b.src_prime[j]].qinv_d, s);
-    constexpr double TOL = 9.094947017729282e-13;                        // 2^-40
-    double f = __builtin_floor(s + TOL);
-    const double g = __builtin_floor(s - TOL);
-    if (f != g && f != 0.0) {
+    for (int j = 0; j < MAXS; j++) s = __builtin_fma(y[j], primes[b.src_prime[j]].qinv_d, s);
+    return conv_quotient_of(s, [&]() {
         double e = 0.0;
 #pragma unroll
         for (int j = 0; j < MAXS; j++) e += y[j] / primes[b.src_prime[j]].qd;
-        f = (double)(int)e;
-    }
-    return (unsigned)(int)f;
+        return e;
+    });
 }
 
 // scaled source residues: as integers and as the doubles that v is formed from
@@ -68,11 +71,10 @@ __device__ __forceinline__ PmSum conv_columns(const u64 (&y)[MAXS], const u64* _
 // columns of products of words below 2^60 with words below 2^50 -> residue modulo a prime below 2^50: with lo = a0 + (a1 mod 2^30) 2^30 below
 // 2^63.3 and hi = a2 + a1 / 2^30 below 2^54 the sum is lo + hi 2^60; its four halves of at most 32 bits are exact doubles, every modular
 // product lies within 0.51 q of zero.
-__device__ __forceinline__ double conv_reduce_f64(const PmSum& s, const PrimeConst& p) {
+__device__ __forceinline__ double conv_reduce_f64(const PmSum& s, double q, double qi, double c32, double c60, double c92) {
     const u64 lo = s.a0 + ((u64)((unsigned)s.a1 & PmSum::MASK30) << 30), hi = s.a2 + (s.a1 >> 30);
-    const double q = p.qd, qi = p.qinv_d;
-    double r = (double)(unsigned)lo + mulmod_f64((double)(unsigned)(lo >> 32), p.c32_d, q, qi);
-    r += mulmod_f64((double)(unsigned)hi, p.c60_d, q, qi) + mulmod_f64((double)(unsigned)(hi >> 32), p.c92_d, q, qi);
+    double r = (double)(unsigned)lo + mulmod_f64((double)(unsigned)(lo >> 32), c32, q, qi);
+    r += mulmod_f64((double)(unsigned)hi, c60, q, qi) + mulmod_f64((double)(unsigned)(hi >> 32), c92, q, qi);
     return canon_f64(r, q, qi);                                          // |r| < 2^32 + 1.6 q
 }
 
@@ -86,7 +88,7 @@ __device__ __forceinline__ u64 conv_target(const u64 (&y)[MAXS], const ConvBlock
         if (centred) r += pr.q - b.sub_out[k];
         return ar.canonical(r);
     } else {
-        double r = conv_reduce_f64(s, pr);
+        double r = conv_reduce_f64(s, pr.qd, pr.qinv_d, pr.c32_d, pr.c60_d, pr.c92_d);
         if (centred) {
             r -= exact_u2d(b.sub_out[k]);
             r = r < 0.0 ? r + pr.qd : r;

@@ -202,6 +202,10 @@ extern "C" int ckks_mult_23(ckks_ctx* c, uint64_t* out, const uint64_t* c1, cons
     u64* axbx = (u64*)work;
     u64* axax = axbx + N * L1;
     u64* bxbx = axax + N * L1;
+    bool lines = false;
+    if (modUp_QjtoT_temp && exProduct_T_temp &&
+        (rc = launch_mult_lines(c, out, c1, c2, rlk, l, (uint64_t*)axax, modUp_QjtoT_temp, exProduct_T_temp, &lines))) return rc;
+    if (lines) return CKKS_OK;
     hipLaunchKernelGGL(tensor_kernel, dim3(N / THREADS, l + 1), dim3(THREADS), 0, c->stream, axbx, axax, bxbx, (const u64*)c1, (const u64*)c2,
                        (const u64*)c1 + N * L1, (const u64*)c2 + N * L1, c->d_primes, N, K);
     CKKS_HIP_TRY(hipGetLastError());
@@ -228,6 +232,11 @@ extern "C" int ckks_rotate_23(ckks_ctx* c, uint64_t* out, const uint64_t* cipher
     const int K = c->K, L1 = c->L + 1;
     u64* a_copy = (u64*)work;                      // the switch leaves its input in the coefficient domain (the reference transforms a back, :571)
     u64* tmp = a_copy + N * L1;                    // cipher_temp_pool
+    bool lines = false;
+    if (modUp_QjtoT_temp && exProduct_T_temp &&
+        (rc = launch_rotate_lines(c, out, cipher, rotkey, H::invmod(H::powmod(5, (u64)rot, 2 * (u64)N), 2 * (u64)N), l, (uint64_t*)a_copy, (uint64_t*)tmp,
+                                  modUp_QjtoT_temp, exProduct_T_temp, &lines))) return rc;
+    if (lines) return CKKS_OK;
     CKKS_HIP_TRY(hipMemcpyAsync(a_copy, cipher, 8 * (size_t)N * (l + 1), hipMemcpyDeviceToDevice, c->stream));
     if ((rc = ckks_keyswitch_23(c, tmp, a_copy, rotkey, l, modUp_QjtoT_temp, exProduct_T_temp, modUp_TtoQj_buffer))) return rc;
     // (tmp.a, tmp.b + b) through the slot permutation with 5^(N/2 - rot) (:582-585): its inverse is 5^rot
@@ -248,6 +257,10 @@ extern "C" int ckks_conjugate_23(ckks_ctx* c, uint64_t* out, const uint64_t* cip
     const long N = c->N;
     const int K = c->K, L1 = c->L + 1;
     u64* a_rev = (u64*)work;
+    bool lines = false;
+    if (modUp_QjtoT_temp && exProduct_T_temp &&
+        (rc = launch_conjugate_lines(c, out, cipher, conjkey, l, (uint64_t*)a_rev, modUp_QjtoT_temp, exProduct_T_temp, &lines))) return rc;
+    if (lines) return CKKS_OK;
     hipLaunchKernelGGL(reverse_kernel, dim3(N / THREADS, l + 1), dim3(THREADS), 0, c->stream, a_rev, (const u64*)cipher, N);                 // :455
     CKKS_HIP_TRY(hipGetLastError());
     if ((rc = ckks_keyswitch_23(c, out, a_rev, conjkey, l, modUp_QjtoT_temp, exProduct_T_temp, modUp_TtoQj_buffer))) return rc;

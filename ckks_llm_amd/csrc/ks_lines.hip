@@ -1,0 +1,229 @@
+// Key switch through the T basis, the operations around it and the rescale as short sequences of line transforms (ntt_fine.hpp,
+// ks_ops.hpp): every step between two transforms runs in a transform's first load or last store, or in the one conversion kernel below.
+//
+//   1 inverse transform of the polynomial to switch   (loads a1 a2 of a product, a of a rotation, a read backwards)
+//   2 forward transform of its digits over T          (loads the conversion Q_j -> T)
+//   3 inverse transform of the sums over T            (loads the external product with the key)
+//   4 T -> [P | Q_l] and ModDown                      (ks_down_kernel)
+//   5 forward transform of the results                (adds the rest of a product, permutes a rotation, adds b)
+//
+// Five launches (up to N = 2^14 and for small levels at 2^15) where the separate steps take ten to fourteen; each saves a write and a read of
+// what it hands over.
+#include "ks_ops.hpp"
+
+namespace ckks {
+
+// ------------------------------------------------------------------------------------------------------------
+// T -> [P | Q_l], centred (BasisConv.cuh:183-254), and ModDown (:257-326) per coefficient: the residues modulo the special primes are formed
+// once per lane and stay in registers, those modulo q_i go straight into (c_q - sum_i [c_p_i (P/p_i)^-1]_p_i (P/p_i)) P^-1 mod q_i.
+// A lane takes the gamma-blocks of its part; the block(s) of the special primes are converted once per part.  All P and Q primes below 2^50,
+// T primes 2^60 - delta.
+// ------------------------------------------------------------------------------------------------------------
+struct KsDownArgs {
+    const u64* in;               // polynomial z at in + z * in_z_stride; limb blk * t_num + j
+    u64* out;                    // q limb i of polynomial z at out + z * out_z_stride + i * N
+    const KsDownTarget* tgt;     // [K + L + 1]
+    const KsDownSource* src;     // [8]
+    long N, in_z_stride, out_z_stride;
+    int K, gamma, t_num, primes, nblocks, parts;      // primes = K + l + 1
+};
+constexpr int KS_DOWN_MAXK = 8;
+template <int MAXS, int MAXK>
+__global__ __launch_bounds__(256) void ks_down_kernel(KsDownArgs a) {
+    const long x = (long)blockIdx.x * 256 + threadIdx.x;
+    const u64* in = a.in + (long)blockIdx.z * a.in_z_stride + x;
+    const KsDownSource* src = table_ptr(a.src);
+    const KsDownTarget* tgt = table_ptr(a.tgt);
+    u64 y[MAXS];
+    double yd[MAXS];
+    unsigned v = 0;
+    int have = -1;                                           // the block that y and v belong to
+    auto block = [&](int blk) {
+        if (blk == have) return;
+        u64 t[MAXS];
+#pragma unroll
+        for (int j = 0; j < MAXS; j++) t[j] = in[(long)(blk * a.t_num + (j < a.t_num ? j : 0)) * a.N];
+        double s = 0.0;
+#pragma unroll
+        for (int j = 0; j < MAXS; j++) {
+            const PmArith ar(src[j].q, src[j].delta);
+            y[j] = ar.canonical(ar.mulmod(t[j] + src[j].add, src[j].hatinv16));
+            yd[j] = (double)y[j];
+            s = __builtin_fma(yd[j], src[j].qinv, s);
+        }
+        v = conv_quotient_of(s, [&]() {
+            double e = 0.0;
+#pragma unroll
+            for (int j = 0; j < MAXS; j++) e += yd[j] / src[j].qd;
+            return e;
+        });
+        have = blk;
+    };
+    // residue modulo a prime of the block, centred
+    auto residue = [&](const KsDownTarget& g) {
+        const PmSum s = conv_columns(y, g.hat, v, g.neg_dmod);
+        const double r = conv_reduce_f64(s, g.qd, g.qinv, g.c32, g.c60, g.c92) - g.sub;
+        return r < 0.0 ? r + g.qd : r;
+    };
+    double rb[MAXK];
+#pragma unroll
+    for (int i = 0; i < MAXK; i++) {
+        rb[i] = 0.0;
+        if (i < a.K) {
+            block(i / a.gamma);
+            const KsDownTarget& g = tgt[i];
+            rb[i] = residue(g);
+            if (a.K > 1) rb[i] = canon_f64(mulmod_f64(rb[i], g.phat[0], g.qd, g.qinv), g.qd, g.qinv);
+        }
+    }
+    const int first = a.K / a.gamma, per = (a.nblocks - first + a.parts - 1) / a.parts;
+    const int b0 = first + (int)blockIdx.y * per, b1 = min(a.nblocks, b0 + per);
+    for (int blk = b0; blk < b1; blk++) {
+        block(blk);
+        const int end = min(a.primes, (blk + 1) * a.gamma);
+        for (int prime = max(a.K, blk * a.gamma); prime < end; prime++) {
+            const KsDownTarget& g = tgt[prime];
+            double acc = 0.0;
+            if (a.K == 1) acc = rb[0];
+            else {
+#pragma unroll
+                for (int i = 0; i < MAXK; i++) acc += mulmod_f64(rb[i], g.phat[i], g.qd, g.qinv);       // at most 8 terms within 0.9 q of zero
+            }
+            const double t = g.qd - canon_f64(acc, g.qd, g.qinv) + residue(g);
+            const double w = mulmod_f64(t, g.pinv, g.qd, g.qinv);
+            a.out[(long)blockIdx.z * a.out_z_stride + (long)(prime - a.K) * a.N + x] = bits52(canon_f64(w, g.qd, g.qinv));
+        }
+    }
+}
+
+// whether the sequence applies: T primes 2^60 - delta, P and Q_l primes on one FP64 back end (0 or 1, returned in *back_end)
+bool ks_lines_apply(const ckks_ctx* c, int l, int* back_end) {
+    if (c->ks_split || c->conv_int || c->arith_mode != 0 || c->ntt_mode != 0 || c->ntt_fine == 4 || c->ev_mid_armed) return false;
+    if (c->logN < 12 || c->logN > 15 || c->t_num <= 0 || c->gamma <= 0 || c->p_num <= 0 || c->p_num > KS_DOWN_MAXK) return false;
+    if ((l + 1 + c->p_num - 1) / c->p_num > c->dnum) return false;               // the key holds fewer digits: the separate steps refuse it
+    const int be = ntt_back_end(c, 0);
+    if (be > 1) return false;
+    for (int i = 0; i < c->p_num + l + 1; i++)
+        if (ntt_back_end(c, i) != be) return false;
+    const ConvPlan& up = c->plan_qj_to_t[l];
+    if (!c->d_down_tgt || up.src_kind != CONV_SRC_F64 || up.tgt_kind != CONV_TGT_PM || up.max_src > 8) return false;
+    *back_end = be;
+    return true;
+}
+
+static NttArgs line_args(const ckks_ctx* c, u64* data, bool inverse, int prime0, int polys, int mods, long poly_mod_len, long batch_stride) {
+    NttArgs a;
+    a.data = data; a.primes = c->d_primes; a.tw = inverse ? c->d_twd_inv : c->d_twd_fwd;
+    a.start_poly_idx = 0; a.start_mod_idx = prime0; a.poly_num = polys; a.mod_num = mods; a.poly_mod_len = (int)poly_mod_len;
+    a.batch_stride_limbs = batch_stride; a.limb_base = 0; a.limbs_total = 0; a.mid = nullptr;
+    return a;
+}
+
+static int down(ckks_ctx* c, u64* out, const u64* ext, int l) {
+    KsDownArgs d;
+    d.in = ext; d.out = out; d.tgt = c->d_down_tgt; d.src = c->d_down_src;
+    d.N = c->N; d.in_z_stride = (long)c->Ri_blockNum * c->t_num * c->N; d.out_z_stride = (long)(c->L + 1) * c->N;
+    d.K = c->K; d.gamma = c->gamma; d.t_num = c->t_num; d.primes = c->K + l + 1; d.nblocks = (d.primes + c->gamma - 1) / c->gamma;
+    // one part per block while the chip has room: a part converts the special primes' block again
+    const int qblocks = d.nblocks - c->K / c->gamma, wgs = (int)(c->N / 256) * 2;
+    d.parts = 1;
+    while (d.parts < qblocks && wgs * d.parts < 3 * c->cu_count) d.parts++;
+    const dim3 g((unsigned)(c->N / 256), d.parts, 2), b(256);
+    if (c->t_num <= 4) {
+        if (c->K <= 4) hipLaunchKernelGGL((ks_down_kernel<4, 4>), g, b, 0, c->stream, d);
+        else hipLaunchKernelGGL((ks_down_kernel<4, 8>), g, b, 0, c->stream, d);
+    } else {
+        if (c->K <= 4) hipLaunchKernelGGL((ks_down_kernel<8, 4>), g, b, 0, c->stream, d);
+        else hipLaunchKernelGGL((ks_down_kernel<8, 8>), g, b, 0, c->stream, d);
+    }
+    CKKS_HIP_TRY(hipGetLastError());
+    return CKKS_OK;
+}
+
+// Steps 1 .. 5 with the first load and the last store given.  d2: the polynomial's coefficients on the way; out: two polynomials of L + 1 limbs
+// (with StoreRotated only the transform's area between its passes).
+template <class AR, class First, class Last>
+static int run(ckks_ctx* c, int back_end, u64* out, u64* d2, const u64* swk, int l, u64* up, u64* ext, const First& first, const Last& last) {
+    const int K = c->K, L1 = c->L + 1, T = c->t_num, RB = c->Ri_blockNum, prime_t = K + L1;
+    const int digits = (l + 1 + K - 1) / K, blocks = (K + l + 1 + c->gamma - 1) / c->gamma;
+    int rc;
+    if ((rc = launch_lines<AR, true>(c, line_args(c, d2, true, K, 1, l + 1, L1, 0), l + 1, back_end, first, StoreLimb()))) return rc;
+    const ConvPlan& plan = c->plan_qj_to_t[l];
+    const NttArgs ua = line_args(c, up, false, prime_t, digits, T, T, 0);
+    auto digits_from = [&](auto ld) {
+        ld.in = d2; ld.blocks = c->d_conv + plan.first; ld.primes = c->d_primes; ld.N = c->N;
+        return launch_lines<PmArith, false>(c, ua, digits * T, 3, ld, StoreLimb());
+    };
+    if (plan.max_src == 1) rc = digits_from(LoadDigits<1>());
+    else if (plan.max_src == 2) rc = digits_from(LoadDigits<2>());
+    else if (plan.max_src <= 4) rc = digits_from(LoadDigits<4>());
+    else rc = digits_from(LoadDigits<8>());
+    if (rc) return rc;
+    LoadExternal ex;
+    ex.up = up; ex.key = swk; ex.N = c->N; ex.key_digit = (long)T * RB; ex.key_z = (long)RB * T * c->dnum; ex.t_num = T; ex.ndigits = digits;
+    if ((rc = launch_lines<PmArith, true>(c, line_args(c, ext, true, prime_t, blocks, T, T, (long)RB * T), 2 * blocks * T, 3, ex, StoreLimb()))) return rc;
+    if ((rc = down(c, out, ext, l))) return rc;
+    return launch_lines<AR, false>(c, line_args(c, out, false, K, 2, l + 1, L1, 0), 2 * (l + 1), back_end, LoadLimb(), last);
+}
+
+template <class First, class Last>
+static int run_on(ckks_ctx* c, int back_end, uint64_t* out, uint64_t* d2, const uint64_t* swk, int l, uint64_t* up, uint64_t* ext, const First& first, const Last& last) {
+    return back_end == 0 ? run<F64Arith>(c, 0, (u64*)out, (u64*)d2, (const u64*)swk, l, (u64*)up, (u64*)ext, first, last)
+                         : run<F64WideArith>(c, 1, (u64*)out, (u64*)d2, (const u64*)swk, l, (u64*)up, (u64*)ext, first, last);
+}
+static bool aligned(std::initializer_list<const void*> ptrs) {
+    for (const void* p : ptrs)
+        if ((uintptr_t)p & 15u) return false;
+    return true;
+}
+
+int launch_keyswitch_lines(ckks_ctx* c, uint64_t* out, uint64_t* d2, const uint64_t* swk, int l, uint64_t* up, uint64_t* ext, bool* done) {
+    int be = 0;
+    *done = ks_lines_apply(c, l, &be) && aligned({out, d2, swk, up, ext});
+    return *done ? run_on(c, be, out, d2, swk, l, up, ext, LoadLimb(), StoreLimb()) : CKKS_OK;
+}
+int launch_mult_lines(ckks_ctx* c, uint64_t* out, const uint64_t* c1, const uint64_t* c2, const uint64_t* swk, int l, uint64_t* d2, uint64_t* up, uint64_t* ext,
+                      bool* done) {
+    int be = 0;
+    const size_t words = (size_t)2 * (c->L + 1) * c->N;
+    // the inputs are read again when the results leave: not where a result overwrites one
+    auto apart = [&](const uint64_t* in) { return out + words <= in || in + words <= out; };
+    *done = ks_lines_apply(c, l, &be) && aligned({out, c1, c2, swk, d2, up, ext}) && apart(c1) && apart(c2);
+    if (!*done) return CKKS_OK;
+    const long N = c->N, L1 = c->L + 1;
+    const u64 *a1 = (const u64*)c1, *a2 = (const u64*)c2;
+    return run_on(c, be, out, d2, swk, l, up, ext, LoadProduct{a1, a2, N}, StoreAddProducts{a1, a1 + N * L1, a2, a2 + N * L1, N});
+}
+int launch_rotate_lines(ckks_ctx* c, uint64_t* out, const uint64_t* cipher, const uint64_t* key, uint64_t pow, int l, uint64_t* d2, uint64_t* tmp, uint64_t* up,
+                        uint64_t* ext, bool* done) {
+    int be = 0;
+    *done = ks_lines_apply(c, l, &be) && aligned({out, cipher, key, d2, tmp, up, ext});
+    if (!*done) return CKKS_OK;
+    const long N = c->N, L1 = c->L + 1;
+    return run_on(c, be, tmp, d2, key, l, up, ext, LoadFrom{(const u64*)cipher, N}, StoreRotated{(u64*)out, (const u64*)cipher + N * L1, pow, N, N * L1, c->logN});
+}
+int launch_conjugate_lines(ckks_ctx* c, uint64_t* out, const uint64_t* cipher, const uint64_t* key, int l, uint64_t* d2, uint64_t* up, uint64_t* ext, bool* done) {
+    int be = 0;
+    *done = ks_lines_apply(c, l, &be) && aligned({out, cipher, key, d2, up, ext});
+    if (!*done) return CKKS_OK;
+    const long N = c->N, L1 = c->L + 1;
+    return run_on(c, be, out, d2, key, l, up, ext, LoadReversed{(const u64*)cipher, N}, StoreAddReversed{(const u64*)cipher + N * L1, N});
+}
+
+// Rescale behind the inverse transform of limb l: one line transform per remaining limb that loads limb l modulo its prime and stores (c - x) q_l^-1.
+int launch_rescale_lines(ckks_ctx* c, uint64_t* cipher, uint64_t* scratch, int l, const uint64_t* inv, bool* done) {
+    *done = false;
+    if (c->ks_split || c->arith_mode != 0 || c->ntt_mode != 0 || c->ntt_fine == 4 || c->ev_mid_armed || c->logN < 12 || c->logN > 15) return CKKS_OK;
+    const int be = ntt_back_end(c, c->K);
+    for (int i = 0; i <= l; i++)
+        if (ntt_back_end(c, c->K + i) != be || be > 1) return CKKS_OK;
+    if (!aligned({cipher, scratch})) return CKKS_OK;
+    const long N = c->N, L1 = c->L + 1;
+    const NttArgs a = line_args(c, (u64*)scratch, false, c->K, 2, l, L1, 0);
+    const LoadReduced ld{(const u64*)cipher + (long)l * N, L1 * N};
+    const StoreRescaled st{(u64*)cipher, (const u64*)inv, L1 * N, N};
+    *done = true;
+    return be == 0 ? launch_lines<F64Arith, false>(c, a, 2 * l, 0, ld, st) : launch_lines<F64WideArith, false>(c, a, 2 * l, 1, ld, st);
+}
+
+}  // namespace ckks

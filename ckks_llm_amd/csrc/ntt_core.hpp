@@ -179,6 +179,7 @@ struct PmArith {
     unsigned delta;
     u64 n_inv16, w1n16;
     static constexpr u64 MASK60 = (1ull << 60) - 1;
+    CKKS_HD PmArith(u64 q_, unsigned delta_) : q(q_), q2(q_ * 2), q8(q_ * 8), delta(delta_), n_inv16(0), w1n16(0) {}      // products only
     CKKS_HD PmArith(const PrimeConst& pc) : q(pc.q), q2(pc.q * 2), q8(pc.q * 8), delta(pc.pm_delta), n_inv16(pc.n_inv << 4), w1n16(pc.w1n << 4) {}
     // x mod q, below 2^60 + 2^30, for any 64-bit x
     CKKS_HD u64 fold(u64 x) const { return (x & MASK60) + (u64)(unsigned)(x >> 60) * delta; }

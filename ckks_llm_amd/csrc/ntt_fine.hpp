@@ -1,0 +1,289 @@
+// Tiles and kernels of the eight-values-per-lane transforms (ntt_lines.hpp) with the operation that produces a transform's input
+// and the one that consumes its output as parameters, so that a step of a longer sequence (a conversion, a product, an addition, a
+// permutation) runs inside the transform's first or last memory access instead of as a launch with a write and a read of its own.
+#pragma once
+#include "ntt_lines.hpp"
+
+namespace ckks {
+
+constexpr int FINE_RL = 3;
+
+// the limb a workgroup works on: where it lies (between the passes as well), its prime, and which polynomial / modulus / batch entry it is
+struct LimbRef {
+    u64* ptr;
+    int prime;
+    unsigned y, j, z;
+};
+__device__ __forceinline__ LimbRef limb_ref(const NttArgs& a, unsigned limb, long N) {
+    LimbRef l;
+    limb += a.limb_base;
+    const unsigned per_mod = a.limbs_total / (unsigned)a.mod_num, r = limb % per_mod;
+    l.j = limb / per_mod;
+    l.y = r % (unsigned)a.poly_num;
+    l.z = r / (unsigned)a.poly_num;
+    l.prime = a.start_mod_idx + (int)l.j;
+    l.ptr = a.data + ((long)l.z * a.batch_stride_limbs + (long)l.y * a.poly_mod_len + a.start_poly_idx + l.j) * N;
+    return l;
+}
+
+// What a transform reads: values at R positions of the limb (forward: gather; inverse: R adjacent ones), in the back end's form.
+struct LoadLimb {
+    template <class AR, int R>
+    __device__ __forceinline__ void gather(const AR& ar, const LimbRef& l, const unsigned (&pos)[R], typename AR::V (&v)[R]) const {
+        u64 x[R];
+#pragma unroll
+        for (int j = 0; j < R; j++) x[j] = l.ptr[pos[j]];
+#pragma unroll
+        for (int j = 0; j < R; j++) v[j] = ar.from_canonical(x[j]);
+    }
+    template <class AR, int R>
+    __device__ __forceinline__ void adjacent(const AR& ar, const LimbRef& l, unsigned p, typename AR::V (&v)[R]) const {
+        u64 x[R];
+        load_adjacent(l.ptr + p, x);
+#pragma unroll
+        for (int j = 0; j < R; j++) v[j] = ar.from_canonical(x[j]);
+    }
+};
+// What a forward transform does with R adjacent results at position p (values as the last round leaves them).
+struct StoreLimb {
+    template <class AR, int R>
+    __device__ __forceinline__ void adjacent(const AR& ar, const LimbRef& l, unsigned p, const typename AR::V (&v)[R]) const {
+        u64 x[R];
+#pragma unroll
+        for (int j = 0; j < R; j++) x[j] = ar.to_canonical_fwd(v[j]);
+        store_adjacent(l.ptr + p, x);
+    }
+};
+
+// SHARED: the tile is one half of a paired launch - what it hands to or takes from the other pass moves as shared accesses
+template <class AR, int SA, int SB, bool INVERSE, bool SHARED, class Load>
+__device__ __forceinline__ void fine_strided_tile(const LimbRef& l, unsigned tile, const typename AR::TW* __restrict__ tw, const AR& ar, typename AR::V* lds,
+                                                  const Load& ld, const TileClaim& claim = TileClaim()) {
+    typedef FineStrided<SA, SB, FINE_RL> F;
+    constexpr int RL = FINE_RL, R = 1 << RL, C0 = line_first<SA, RL>();
+    constexpr long N2 = 1l << SB;
+    const unsigned cl = threadIdx.x % F::CW, u = threadIdx.x / F::CW;
+    u64* col = l.ptr + tile * F::CW + cl;
+    auto at = [&](unsigned p) { return lds + p * F::CW + cl; };
+    typedef LineRound<SA, RL, 0, C0> LR;
+    typename AR::V v[R];
+    if constexpr (!INVERSE) {
+        RoundTw<AR, SA, RL, 0, C0> w;
+        w.load(tw, 1u, u);
+        unsigned pos[R];
+#pragma unroll
+        for (int h = 0; h < LR::GROUPS; h++)
+#pragma unroll
+            for (int j = 0; j < (1 << C0); j++) pos[(h << C0) + j] = LR::pos(LR::group(u, h), j) * (unsigned)N2 + tile * F::CW + cl;
+        ld.gather(ar, l, pos, v);
+        const unsigned raw = claim.start(threadIdx.x);
+        if (!line_fwd<AR, SA, RL>(v, w, tw, 1u, u, ar, at, claim, raw)) return;
+#pragma unroll
+        for (int j = 0; j < R; j++) put<SHARED>(col + (long)(u * R + j) * N2, ar.to_mid_fwd(v[j]));
+    } else {
+        RoundTw<AR, SA, RL, SA - RL, RL> w;
+        w.load(tw, 1u, u);
+        u64 x[R];
+#pragma unroll
+        for (int j = 0; j < R; j++) x[j] = get<SHARED>(col + (long)(u * R + j) * N2);
+        const unsigned counted = claim.start(threadIdx.x);
+#pragma unroll
+        for (int j = 0; j < R; j++) v[j] = ar.from_mid(x[j]);
+        line_inv<AR, SA, RL, true>(v, w, tw, 1u, u, ar, at);
+        line_inv_last<AR, SA, RL>(v, x, ar);
+#pragma unroll
+        for (int h = 0; h < LR::GROUPS; h++)
+#pragma unroll
+            for (int j = 0; j < (1 << C0); j++) col[LR::pos(LR::group(u, h), j) * N2] = x[(h << C0) + j];
+        claim.publish(threadIdx.x, counted);
+    }
+}
+
+// Op: what the inverse transform loads (Load) or what the forward transform stores (Store)
+template <class AR, int SA, int SB, bool INVERSE, bool SHARED, class Op>
+__device__ __forceinline__ void fine_row_tile(const LimbRef& l, unsigned tile, const typename AR::TW* __restrict__ tw, const AR& ar, typename AR::V* lds,
+                                              const Op& op, const TileClaim& claim = TileClaim()) {
+    typedef FineRow<SA, SB, FINE_RL> F;
+    constexpr int RL = FINE_RL, R = 1 << RL, C0 = line_first<SB, RL>(), N1 = 1 << SA;
+    constexpr long N2 = 1l << SB;
+    const unsigned u = threadIdx.x % F::U, rl = threadIdx.x / F::U;
+    const unsigned row = tile * F::ROWS + rl, tw_off = N1 + row;
+    u64* rp = l.ptr + row * N2;
+    typename AR::V* lrow = lds + rl * F::PITCH;
+    auto at = [&](unsigned p) { return lrow + padded((int)p); };
+    typedef LineRound<SB, RL, 0, C0> LR;
+    typename AR::V v[R];
+    if constexpr (!INVERSE) {
+        RoundTw<AR, SB, RL, 0, C0> w;
+        w.load(tw, tw_off, u);
+        u64 x[R];
+#pragma unroll
+        for (int h = 0; h < LR::GROUPS; h++)
+#pragma unroll
+            for (int j = 0; j < (1 << C0); j++) x[(h << C0) + j] = get<SHARED>(rp + LR::pos(LR::group(u, h), j));
+        const unsigned counted = claim.start(threadIdx.x);
+#pragma unroll
+        for (int j = 0; j < R; j++) v[j] = ar.from_mid(x[j]);
+        line_fwd<AR, SB, RL>(v, w, tw, tw_off, u, ar, at);
+        op.adjacent(ar, l, row * (unsigned)N2 + u * R, v);
+        claim.publish(threadIdx.x, counted);
+    } else {
+        RoundTw<AR, SB, RL, SB - RL, RL> w;
+        w.load(tw, tw_off, u);
+        op.adjacent(ar, l, row * (unsigned)N2 + u * R, v);
+        const unsigned raw = claim.start(threadIdx.x);
+        if (!line_inv<AR, SB, RL, false>(v, w, tw, tw_off, u, ar, at, claim, raw)) return;
+#pragma unroll
+        for (int h = 0; h < LR::GROUPS; h++)
+#pragma unroll
+            for (int j = 0; j < (1 << C0); j++) put<SHARED>(rp + LR::pos(LR::group(u, h), j), ar.to_mid_inv(v[(h << C0) + j]));
+    }
+}
+
+template <int SA, int SB> constexpr int fine_lds_words() {
+    return FineStrided<SA, SB, FINE_RL>::LDS_WORDS > FineRow<SA, SB, FINE_RL>::LDS_WORDS ? FineStrided<SA, SB, FINE_RL>::LDS_WORDS : FineRow<SA, SB, FINE_RL>::LDS_WORDS;
+}
+template <class AR, int SA, int SB, bool INVERSE, class Load>
+__global__ __launch_bounds__((FineStrided<SA, SB, FINE_RL>::THREADS)) void fine_strided_kernel(NttArgs a, Load ld) {
+    constexpr long N = 1l << (SA + SB);
+    __shared__ typename AR::V lds[FineStrided<SA, SB, FINE_RL>::LDS_WORDS];
+    const LimbRef l = limb_ref(a, blockIdx.y, N);
+    const AR ar(a.primes[l.prime]);
+    fine_strided_tile<AR, SA, SB, INVERSE, false>(l, blockIdx.x, (const typename AR::TW*)a.tw + (long)l.prime * N, ar, lds, ld);
+}
+template <class AR, int SA, int SB, bool INVERSE, class Op>
+__global__ __launch_bounds__((FineRow<SA, SB, FINE_RL>::THREADS)) void fine_row_kernel(NttArgs a, Op op) {
+    constexpr long N = 1l << (SA + SB);
+    __shared__ typename AR::V lds[FineRow<SA, SB, FINE_RL>::LDS_WORDS];
+    const LimbRef l = limb_ref(a, blockIdx.y, N);
+    const AR ar(a.primes[l.prime]);
+    fine_row_tile<AR, SA, SB, INVERSE, false>(l, blockIdx.x, (const typename AR::TW*)a.tw + (long)l.prime * N, ar, lds, op);
+}
+// both passes in one launch of one workgroup per (limb, tile)
+template <class AR, int SA, int SB, bool INVERSE, class Load, class Store>
+__global__ __launch_bounds__((FineStrided<SA, SB, FINE_RL>::THREADS)) void fine_pair_kernel(NttArgs a, PairArgs p, Load ld, Store st) {
+    constexpr unsigned TILES = FineStrided<SA, SB, FINE_RL>::TILES;
+    constexpr long N = 1l << (SA + SB);
+    __shared__ typename AR::V lds[fine_lds_words<SA, SB>()];
+    __shared__ unsigned go;
+    unsigned limb_id, tile;
+    pair_block(p, blockIdx.x, TILES, limb_id, tile);
+    if (limb_id >= p.limbs) return;                                             // uniform over the workgroup
+    const LimbRef l = limb_ref(a, limb_id, N);
+    const AR ar(a.primes[l.prime]);
+    const typename AR::TW* __restrict__ tw = (const typename AR::TW*)a.tw + (long)l.prime * N;
+    pair_run<TILES>(p, limb_id, tile, &go, p.steal != 0,
+                    [&](unsigned t, const TileClaim& claim) {
+                        if constexpr (!INVERSE) fine_strided_tile<AR, SA, SB, false, true>(l, t, tw, ar, lds, ld, claim);
+                        else fine_row_tile<AR, SA, SB, true, true>(l, t, tw, ar, lds, ld, claim);
+                    },
+                    [&](unsigned t, const TileClaim& out) {
+                        if constexpr (!INVERSE) fine_row_tile<AR, SA, SB, false, true>(l, t, tw, ar, lds, st, out);
+                        else fine_strided_tile<AR, SA, SB, true, true>(l, t, tw, ar, lds, ld, out);
+                    });
+}
+
+// whole limb: values per lane chosen so that a workgroup has at most 1024 lanes
+template <int S> constexpr int whole_rl() { return S <= 13 ? 3 : 4; }
+template <class AR, int S, bool INVERSE, class Load, class Store>
+__global__ __launch_bounds__((FineWhole<S, whole_rl<S>()>::THREADS)) void fine_whole_kernel(NttArgs a, Load ld, Store st) {
+    constexpr int RL = whole_rl<S>(), R = 1 << RL, C0 = line_first<S, RL>();
+    typedef FineWhole<S, RL> F;
+    constexpr long N = 1l << S;
+    typedef typename AR::TW TW;
+    __shared__ typename AR::V lds[F::LDS_WORDS];
+    const LimbRef l = limb_ref(a, blockIdx.x, N);
+    const AR ar(a.primes[l.prime]);
+    const TW* __restrict__ tw = (const TW*)a.tw + (long)l.prime * N;
+    const unsigned u = threadIdx.x;
+    auto at = [&](unsigned p) { return lds + padded((int)p); };
+    typedef LineRound<S, RL, 0, C0> LR;
+    typename AR::V v[R];
+    if constexpr (!INVERSE) {
+        RoundTw<AR, S, RL, 0, C0> w;
+        w.load(tw, 1u, u);
+        unsigned pos[R];
+#pragma unroll
+        for (int h = 0; h < LR::GROUPS; h++)
+#pragma unroll
+            for (int j = 0; j < (1 << C0); j++) pos[(h << C0) + j] = LR::pos(LR::group(u, h), j);
+        ld.gather(ar, l, pos, v);
+        line_fwd<AR, S, RL>(v, w, tw, 1u, u, ar, at);
+        st.adjacent(ar, l, u * R, v);
+    } else {
+        RoundTw<AR, S, RL, S - RL, RL> w;
+        w.load(tw, 1u, u);
+        ld.adjacent(ar, l, u * R, v);
+        line_inv<AR, S, RL, true>(v, w, tw, 1u, u, ar, at);
+        u64 x[R];
+        line_inv_last<AR, S, RL>(v, x, ar);
+#pragma unroll
+        for (int h = 0; h < LR::GROUPS; h++)
+#pragma unroll
+            for (int j = 0; j < (1 << C0); j++) l.ptr[LR::pos(LR::group(u, h), j)] = x[(h << C0) + j];
+    }
+}
+
+// ---- launches ----
+PairArgs pair_args(const ckks_ctx* c, int limbs);
+unsigned pair_blocks(int limbs, unsigned tiles);
+int pair_region(ckks_ctx* c, int limbs);                    // -1: no protocol words for this call (see ntt_fine.hip)
+
+template <class AR, int S, bool INVERSE, class Load, class Store>
+int launch_whole(ckks_ctx* c, const NttArgs& a, int limbs, const Load& ld, const Store& st) {
+    const dim3 g((unsigned)limbs), b(FineWhole<S, whole_rl<S>()>::THREADS);
+    hipLaunchKernelGGL((fine_whole_kernel<AR, S, INVERSE, Load, Store>), g, b, 0, c->stream, a, ld, st);
+    CKKS_HIP_TRY(hipGetLastError());
+    return CKKS_OK;
+}
+template <class AR, int SA, int SB, bool INVERSE, class Load, class Store>
+int launch_fine(ckks_ctx* c, const NttArgs& a, int limbs, bool pair, const Load& ld, const Store& st) {
+    typedef FineStrided<SA, SB, FINE_RL> FS;
+    typedef FineRow<SA, SB, FINE_RL> FR;
+    const int region = pair ? pair_region(c, limbs) : -1;
+    if (region >= 0) {
+        PairArgs p = pair_args(c, limbs);
+        p.done += (size_t)region * PAIR_WORD_STRIDE;
+        p.spread = 0;                                   // a limb's tiles on one XCD: spread over all of them 20.2 us against 16.0 (N = 2^15, 48 limbs)
+        const dim3 g(pair_blocks(limbs, FS::TILES)), b(FS::THREADS);
+        hipLaunchKernelGGL((fine_pair_kernel<AR, SA, SB, INVERSE, Load, Store>), g, b, 0, c->stream, a, p, ld, st);
+    } else {
+        const dim3 gs(FS::TILES, limbs), bs(FS::THREADS), gr(FR::TILES, limbs), br(FR::THREADS);
+        if constexpr (!INVERSE) {
+            hipLaunchKernelGGL((fine_strided_kernel<AR, SA, SB, false, Load>), gs, bs, 0, c->stream, a, ld);
+            hipLaunchKernelGGL((fine_row_kernel<AR, SA, SB, false, Store>), gr, br, 0, c->stream, a, st);
+        } else {
+            hipLaunchKernelGGL((fine_row_kernel<AR, SA, SB, true, Load>), gr, br, 0, c->stream, a, ld);
+            hipLaunchKernelGGL((fine_strided_kernel<AR, SA, SB, true, LoadLimb>), gs, bs, 0, c->stream, a, LoadLimb());
+        }
+    }
+    CKKS_HIP_TRY(hipGetLastError());
+    return CKKS_OK;
+}
+// A transform of `limbs` limbs with its first load and (forward) last store given, N = 2^12 .. 2^16: whole limbs at 2^12 and for the larger
+// batches at 2^13, otherwise two passes, paired where ntt_fine_form pairs a plain transform of that size.
+template <class AR, bool INVERSE, class Load, class Store>
+int launch_lines(ckks_ctx* c, NttArgs a, int limbs, int back_end, const Load& ld, const Store& st) {
+    a.limb_base = 0;
+    a.limbs_total = (unsigned)limbs;
+    a.mid = nullptr;
+    const int form = ntt_fine_form(c, limbs, back_end);
+    switch (c->logN) {
+        case 12: return launch_whole<AR, 12, INVERSE>(c, a, limbs, ld, st);
+        case 13:
+            if (form == 1) return launch_whole<AR, 13, INVERSE>(c, a, limbs, ld, st);
+            if (form == 5) return launch_fine<AR, 6, 7, INVERSE>(c, a, limbs, true, ld, st);
+            return launch_fine<AR, 7, 6, INVERSE>(c, a, limbs, form == 3, ld, st);
+        case 14:
+            if (form == 5) return launch_fine<AR, 6, 8, INVERSE>(c, a, limbs, true, ld, st);
+            return launch_fine<AR, 7, 7, INVERSE>(c, a, limbs, form == 3, ld, st);
+        case 15:
+            if (form == 5) return launch_fine<AR, 7, 8, INVERSE>(c, a, limbs, true, ld, st);
+            return launch_fine<AR, 8, 7, INVERSE>(c, a, limbs, form == 3, ld, st);
+        case 16: return launch_fine<AR, 8, 8, INVERSE>(c, a, limbs, form == 3, ld, st);
+    }
+    set_error("NTT: no line form at this ring size");
+    return CKKS_E_INVALID;
+}
+
+}  // namespace ckks

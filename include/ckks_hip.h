@@ -108,7 +108,7 @@ int ckks_ctx_set_ntt_chain(ckks_ctx* ctx, int skew, int spin_max);
  *   "conv_int"        basis conversions into primes below 2^50 accumulate in 128-bit integers instead of FP64
  *   "ntt_no_reverse"  the second launch of a two-launch transform takes the limbs in forward order
  *   "ntt_fine"        value = 1: a limb per workgroup (N = 2^12 .. 2^14), 2: two passes with eight values per lane, 3: the same paired in one
- *                     launch (N >= 2^13), wherever the form exists; 4: none of them
+ *                     launch (N >= 2^13), 5: paired with tiles of half the size (N = 2^13 .. 2^15), wherever the form exists; 4: none of them
  *   "ntt_chunk"       value = limbs per trip through the inter-pass buffer of a two-launch transform (0: the whole batch) */
 int ckks_ctx_set_option(ckks_ctx* ctx, const char* name, long value);
 /* Order of work of the chained transform, for tests: slot `slot` of a chain of `tiles` workgroups per pass -> pass (0 / 1),

@@ -7,6 +7,7 @@ import pytest
 from ckks_llm_amd import CkksError, Ciphertext, Context_23, DeviceBuffer, Plaintext, Scheme_23, SecretKey
 from oracle import oracle_py as O
 from tests.gpu_common import Pair, to_dev, from_dev
+from tests.helpers import limbs_uniform
 from tests.params import REF_PARAMS
 
 pytestmark = pytest.mark.gpu
@@ -303,3 +304,54 @@ def test_in_place_and_derived_members_leave_the_same_words():
     assert a2.l == L - 3 and np.array_equal(words(a2), want.reshape(2, L + 1, N)[:, : L - 2])
     prod = float(np.prod([float(x) for x in ctx.qVec[L - 2:]]))
     assert abs(a2.scale * prod / a.scale - 1) < 1e-9
+
+
+@pytest.mark.parametrize("params,logN", [(13, 12), (13, 13), (14, 13), (14, 14), (15, 14), (15, 15)])
+def test_operations_as_line_transforms(params, logN):
+    """mult_23, leftRotate_23, conjugate_23, keyswitch_23 and rescaleAndEqual at the ring sizes where each step of them runs inside a
+    transform's first load or last store: uniform keys and operands (largest residues in some columns), at the top level, in the middle
+    (a digit cut by the level) and at the bottom; against the oracle, and against the separate launches for a product that overwrites an
+    operand."""
+    pair = ref_pair(params, logN)
+    orc, dev, L_ = pair.orc, pair.dev, pair.dev.L_
+    N, K, L, T, RB, dnum = pair.N, orc.K, orc.L, orc.t_num, orc.Ri_blockNum, orc.dnum
+    L1 = L + 1
+    key = limbs_uniform(3, orc.t, 2 * dnum * RB, N)
+    cts = [limbs_uniform(4 + i, orc.q, 2, N) for i in range(2)]
+    for j, q in enumerate(orc.q):
+        key[:, :, 5] = np.array(orc.t, dtype=np.uint64) - 1
+        cts[0][:, j, 5:8] = q - 1
+        cts[1][:, j, 6:9] = q - 1
+    d_key, d_c = to_dev(key), [to_dev(c) for c in cts]
+    work, up = DeviceBuffer(8 * N * L1 * 3), DeviceBuffer(8 * N * T * orc.Qj_blockNum)
+    ext, buf = DeviceBuffer(8 * N * T * RB * 2), DeviceBuffer(8 * N * T * RB * 2)
+    scratch = DeviceBuffer(8 * N * L1 * 2)
+    flat, zero = key.reshape(-1), np.zeros((2, L1, N), dtype=np.uint64)
+    for l in sorted({L, max(1, L // 2), 1}):
+        want = zero.copy()
+        orc.mult_23(want.reshape(-1), cts[0].reshape(-1), cts[1].reshape(-1), flat, l)
+        d_out = to_dev(zero)
+        assert L_.ckks_mult_23(dev.h, d_out.ptr, d_c[0].ptr, d_c[1].ptr, d_key.ptr, l, work.ptr, up.ptr, ext.ptr, buf.ptr) == 0
+        assert np.array_equal(from_dev(d_out, want.shape)[:, :l + 1], want[:, :l + 1]), ("mult", l)
+        d_alias = to_dev(cts[0])
+        assert L_.ckks_mult_23(dev.h, d_alias.ptr, d_alias.ptr, d_c[1].ptr, d_key.ptr, l, work.ptr, up.ptr, ext.ptr, buf.ptr) == 0
+        assert np.array_equal(from_dev(d_alias, want.shape)[:, :l + 1], want[:, :l + 1]), ("mult in place", l)
+        orc.rescaleAndEqual(want.reshape(-1), l)
+        dev.rescaleAndEqual(d_out, scratch, l)
+        assert np.array_equal(from_dev(d_out, want.shape)[:, :l], want[:, :l]), ("rescale", l)
+        for rot in (1, N // 2 - 3):
+            want = zero.copy()
+            orc.leftRotate_23(want.reshape(-1), cts[0].reshape(-1), flat, rot, l)
+            assert L_.ckks_rotate_23(dev.h, d_out.ptr, d_c[0].ptr, d_key.ptr, rot, l, work.ptr, up.ptr, ext.ptr, buf.ptr) == 0
+            assert np.array_equal(from_dev(d_out, want.shape)[:, :l + 1], want[:, :l + 1]), ("rot", rot, l)
+        want = zero.copy()
+        orc.conjugate_23(want.reshape(-1), cts[0].reshape(-1), flat, l)
+        assert L_.ckks_conjugate_23(dev.h, d_out.ptr, d_c[0].ptr, d_key.ptr, l, work.ptr, up.ptr, ext.ptr, buf.ptr) == 0
+        assert np.array_equal(from_dev(d_out, want.shape)[:, :l + 1], want[:, :l + 1]), ("conj", l)
+        want = zero.copy()
+        d2 = np.ascontiguousarray(cts[0][0])
+        orc.keyswitch_23(want.reshape(-1), d2.copy().reshape(-1), flat, l)
+        dev.keyswitch_23(d_out, to_dev(d2), d_key, l, up, ext, buf)
+        assert np.array_equal(from_dev(d_out, want.shape)[:, :l + 1], want[:, :l + 1]), ("keyswitch", l)
+        for c, d in zip(cts, d_c):
+            assert np.array_equal(from_dev(d, c.shape), c)                                    # operands are left as they were

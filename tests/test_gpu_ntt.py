@@ -140,7 +140,7 @@ def test_pseudo_mersenne_backend_at_its_range_ends(logN):
             buf.free()
 
 
-@pytest.mark.parametrize("logN,form", [(12, 1), (13, 1), (14, 1), (13, 2), (14, 2), (15, 2), (16, 2), (13, 3), (14, 3), (15, 3), (16, 3)])
+@pytest.mark.parametrize("logN,form", [(12, 1), (13, 1), (14, 1), (13, 2), (14, 2), (15, 2), (16, 2), (13, 3), (14, 3), (15, 3), (16, 3), (13, 5), (14, 5), (15, 5)])
 def test_eight_values_per_lane_forms_match_oracle(logN, form):
     """Whole limbs in one workgroup, two passes with eight values per lane and the same paired in one launch, for 36-, 49- and 60-bit
     primes and the general integers (a 55-bit one), with padding limbs and start indices, in both directions; largest residues
@@ -158,7 +158,7 @@ def test_eight_values_per_lane_forms_match_oracle(logN, form):
         if top:
             for j in range(mods):
                 data[:, 1 + j] = primes[first + j] - 1
-        for spin, steal in ((None, True), (0, True), (0, False)) if form == 3 else ((None, True),):
+        for spin, steal in ((None, True), (0, True), (0, False)) if form in (3, 5) else ((None, True),):
             pair.dev.set_ntt_chain(0, -1 if spin is None else spin)
             pair.dev.set_option("pair_no_steal", 0 if steal else 1)
             for inverse in (False, True):
