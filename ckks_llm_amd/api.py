@@ -102,6 +102,7 @@ class Context_23:
             p, q, t, gamma = r["p"], r["q"], r["t"], r["gamma"]
             self.precision = 1 << 36 if logN < 15 else 1 << 49               # Params.cuh:15, 36, 58, 85
         self.slots = 1 << self.logslots
+        self._stream, self._scratch = None, []
         self.L_ = load_library()
         self.logN, self.N = logN, 1 << logN
         self.pVec, self.qVec, self.tVec = list(p), list(q), list(t)
@@ -159,6 +160,7 @@ class Context_23:
 
     def set_stream(self, stream_handle):
         _check(self.L_.ckks_set_stream(self.h, stream_handle), "ckks_set_stream")
+        self._stream = stream_handle
 
     def sync(self):
         _check(self.L_.ckks_sync(), "ckks_sync")
@@ -312,10 +314,27 @@ class Context_23:
 
     def decode_coeffs(self, msg, vals, is_bitRev=False):
         """vals: N device doubles (written)."""
-        scratch = DeviceBuffer(8 * self.N * (msg.l + 1))
+        scratch = self._take_scratch(8 * self.N * (msg.l + 1))
         _check(self.L_.ckks_decode_coeffs(self.h, _addr(vals), _addr(msg.mx_device), scratch.ptr, float(msg.scale), msg.slots,
                                           1 if is_bitRev else 0, msg.l), "ckks_decode_coeffs")
-        scratch.free()
+        if not self._stream and len(self._scratch) < 2:
+            self._scratch.append(scratch)
+        else:
+            scratch.free()
+
+    def _take_scratch(self, nbytes):
+        """A work area of at least nbytes.  On the null stream, whose order keeps one call's use apart from the next and from every
+        copy of the results, up to two are kept between calls (a call holds its own while it issues its launches): freeing one waits
+        for the device, which a 70 us call paid for every time.  On any other stream a call has an area of its own."""
+        if not self._stream:
+            try:
+                buf = self._scratch.pop()
+                if buf.nbytes >= nbytes:
+                    return buf
+            except IndexError:
+                pass
+            nbytes = max(nbytes, 8 * self.N * (self.L + 1))
+        return DeviceBuffer(nbytes)
 
 
 class Plaintext:

@@ -204,6 +204,10 @@ int launch_rotate_lines(ckks_ctx* c, uint64_t* out, const uint64_t* cipher, cons
                         uint64_t* up, uint64_t* ext, bool* done);
 int launch_conjugate_lines(ckks_ctx* c, uint64_t* out, const uint64_t* cipher, const uint64_t* key, int l, uint64_t* d2, uint64_t* up, uint64_t* ext,
                            bool* done);
+// The client's steps inside their transforms (scheme_lines.hip); *done = false: not applicable, nothing launched.
+int launch_encode_lines(ckks_ctx* c, uint64_t* mx, const double* vals, long scale, int l, bool* done);
+int launch_encrypt_lines(ckks_ctx* c, uint64_t* cipher, const uint64_t* mx, const uint64_t* pk, const uint8_t* random, uint64_t* scratch, int l, bool* done);
+int launch_coefficients_lines(ckks_ctx* c, uint64_t* out, const uint64_t* mx, int l, bool* done);
 int launch_rescale_lines(ckks_ctx* c, uint64_t* cipher, uint64_t* scratch, int l, const uint64_t* inv, bool* done);
 // The maps modUpTtoPQl_23, modUpQjtoT_23 and modDownPQltoQl_23 on `batch` polynomials with strides of the caller's, in words.  The ModDown may
 // write over its own Q limbs (out = in + p_num limbs): a coefficient's output only depends on words that no other output overwrites.

@@ -111,14 +111,6 @@ bool ks_lines_apply(const ckks_ctx* c, int l, int* back_end) {
     return true;
 }
 
-static NttArgs line_args(const ckks_ctx* c, u64* data, bool inverse, int prime0, int polys, int mods, long poly_mod_len, long batch_stride) {
-    NttArgs a;
-    a.data = data; a.primes = c->d_primes; a.tw = inverse ? c->d_twd_inv : c->d_twd_fwd;
-    a.start_poly_idx = 0; a.start_mod_idx = prime0; a.poly_num = polys; a.mod_num = mods; a.poly_mod_len = (int)poly_mod_len;
-    a.batch_stride_limbs = batch_stride; a.limb_base = 0; a.limbs_total = 0; a.mid = nullptr;
-    return a;
-}
-
 static int down(ckks_ctx* c, u64* out, const u64* ext, int l) {
     KsDownArgs d;
     d.in = ext; d.out = out; d.tgt = c->d_down_tgt; d.src = c->d_down_src;
@@ -171,15 +163,9 @@ static int run_on(ckks_ctx* c, int back_end, uint64_t* out, uint64_t* d2, const 
     return back_end == 0 ? run<F64Arith>(c, 0, (u64*)out, (u64*)d2, (const u64*)swk, l, (u64*)up, (u64*)ext, first, last)
                          : run<F64WideArith>(c, 1, (u64*)out, (u64*)d2, (const u64*)swk, l, (u64*)up, (u64*)ext, first, last);
 }
-static bool aligned(std::initializer_list<const void*> ptrs) {
-    for (const void* p : ptrs)
-        if ((uintptr_t)p & 15u) return false;
-    return true;
-}
-
 int launch_keyswitch_lines(ckks_ctx* c, uint64_t* out, uint64_t* d2, const uint64_t* swk, int l, uint64_t* up, uint64_t* ext, bool* done) {
     int be = 0;
-    *done = ks_lines_apply(c, l, &be) && aligned({out, d2, swk, up, ext});
+    *done = ks_lines_apply(c, l, &be) && words16({out, d2, swk, up, ext});
     return *done ? run_on(c, be, out, d2, swk, l, up, ext, LoadLimb(), StoreLimb()) : CKKS_OK;
 }
 int launch_mult_lines(ckks_ctx* c, uint64_t* out, const uint64_t* c1, const uint64_t* c2, const uint64_t* swk, int l, uint64_t* d2, uint64_t* up, uint64_t* ext,
@@ -188,7 +174,7 @@ int launch_mult_lines(ckks_ctx* c, uint64_t* out, const uint64_t* c1, const uint
     const size_t words = (size_t)2 * (c->L + 1) * c->N;
     // the inputs are read again when the results leave: not where a result overwrites one
     auto apart = [&](const uint64_t* in) { return out + words <= in || in + words <= out; };
-    *done = ks_lines_apply(c, l, &be) && aligned({out, c1, c2, swk, d2, up, ext}) && apart(c1) && apart(c2);
+    *done = ks_lines_apply(c, l, &be) && words16({out, c1, c2, swk, d2, up, ext}) && apart(c1) && apart(c2);
     if (!*done) return CKKS_OK;
     const long N = c->N, L1 = c->L + 1;
     const u64 *a1 = (const u64*)c1, *a2 = (const u64*)c2;
@@ -197,14 +183,14 @@ int launch_mult_lines(ckks_ctx* c, uint64_t* out, const uint64_t* c1, const uint
 int launch_rotate_lines(ckks_ctx* c, uint64_t* out, const uint64_t* cipher, const uint64_t* key, uint64_t pow, int l, uint64_t* d2, uint64_t* tmp, uint64_t* up,
                         uint64_t* ext, bool* done) {
     int be = 0;
-    *done = ks_lines_apply(c, l, &be) && aligned({out, cipher, key, d2, tmp, up, ext});
+    *done = ks_lines_apply(c, l, &be) && words16({out, cipher, key, d2, tmp, up, ext});
     if (!*done) return CKKS_OK;
     const long N = c->N, L1 = c->L + 1;
     return run_on(c, be, tmp, d2, key, l, up, ext, LoadFrom{(const u64*)cipher, N}, StoreRotated{(u64*)out, (const u64*)cipher + N * L1, pow, N, N * L1, c->logN});
 }
 int launch_conjugate_lines(ckks_ctx* c, uint64_t* out, const uint64_t* cipher, const uint64_t* key, int l, uint64_t* d2, uint64_t* up, uint64_t* ext, bool* done) {
     int be = 0;
-    *done = ks_lines_apply(c, l, &be) && aligned({out, cipher, key, d2, up, ext});
+    *done = ks_lines_apply(c, l, &be) && words16({out, cipher, key, d2, up, ext});
     if (!*done) return CKKS_OK;
     const long N = c->N, L1 = c->L + 1;
     return run_on(c, be, out, d2, key, l, up, ext, LoadReversed{(const u64*)cipher, N}, StoreAddReversed{(const u64*)cipher + N * L1, N});
@@ -217,7 +203,7 @@ int launch_rescale_lines(ckks_ctx* c, uint64_t* cipher, uint64_t* scratch, int l
     const int be = ntt_back_end(c, c->K);
     for (int i = 0; i <= l; i++)
         if (ntt_back_end(c, c->K + i) != be || be > 1) return CKKS_OK;
-    if (!aligned({cipher, scratch})) return CKKS_OK;
+    if (!words16({cipher, scratch})) return CKKS_OK;
     const long N = c->N, L1 = c->L + 1;
     const NttArgs a = line_args(c, (u64*)scratch, false, c->K, 2, l, L1, 0);
     const LoadReduced ld{(const u64*)cipher + (long)l * N, L1 * N};

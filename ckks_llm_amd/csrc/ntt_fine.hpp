@@ -2,6 +2,8 @@
 // and the one that consumes its output as parameters, so that a step of a longer sequence (a conversion, a product, an addition, a
 // permutation) runs inside the transform's first or last memory access instead of as a launch with a write and a read of its own.
 #pragma once
+#include <initializer_list>
+
 #include "ntt_lines.hpp"
 
 namespace ckks {
@@ -284,6 +286,22 @@ int launch_lines(ckks_ctx* c, NttArgs a, int limbs, int back_end, const Load& ld
     }
     set_error("NTT: no line form at this ring size");
     return CKKS_E_INVALID;
+}
+
+// arguments of a transform of `polys` polynomials of `mods` limbs from prime0 on
+inline NttArgs line_args(const ckks_ctx* c, u64* data, bool inverse, int prime0, int polys, int mods, long poly_mod_len, long batch_stride) {
+    NttArgs a;
+    a.data = data; a.primes = c->d_primes; a.tw = inverse ? c->d_twd_inv : c->d_twd_fwd;
+    a.start_poly_idx = 0; a.start_mod_idx = prime0; a.poly_num = polys; a.mod_num = mods; a.poly_mod_len = (int)poly_mod_len;
+    a.batch_stride_limbs = batch_stride; a.limb_base = 0; a.limbs_total = 0; a.mid = nullptr;
+    return a;
+}
+
+// whether all of them may be accessed in 16-byte pieces
+inline bool words16(std::initializer_list<const void*> ptrs) {
+    for (const void* p : ptrs)
+        if ((uintptr_t)p & 15u) return false;
+    return true;
 }
 
 }  // namespace ckks

@@ -9,6 +9,7 @@
 // kernel, the batched transforms, and one combining kernel.  All of it is HBM-bound streaming work: every lane handles one
 // coefficient of every limb of a call, 8-byte accesses coalesced along the coefficient index.
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -16,9 +17,22 @@
 
 #include "context.hpp"
 #include "host_math.hpp"
+#include "samplers.hpp"
 
 using namespace ckks;
 namespace H = ckks_host;
+
+const GaussSteps& ckks::gauss_steps() {
+    static GaussSteps g = [] {
+        GaussSteps s;
+        for (int k = 1; k <= 19; k++) {
+            const double tail = 0.5 * std::erfc(((double)k / 3.2) / std::sqrt(2.0));
+            s.thr[k - 1] = (uint32_t)(4294967296.0 - std::floor(4294967296.0 * tail + 0.5));
+        }
+        return s;
+    }();
+    return g;
+}
 
 namespace {
 
@@ -70,34 +84,6 @@ __global__ __launch_bounds__(THREADS) void salsa20_kernel(uint8_t* out, size_t n
 // ---------------------------------------------------------------------------------------------------------------------------------
 // conversions of random bytes
 // ---------------------------------------------------------------------------------------------------------------------------------
-// Steps of the discrete Gaussian as thresholds on the 32-bit word: value >= k  <=>  u >= thr[k-1], k = 1..19; the negative side is
-// the mirror image u -> ~u.  thr[k-1] = 2^32 - floor(2^32 * Q(k / 3.2) + 0.5) with Q the upper normal tail, i.e. the probability of a
-// word is taken at the middle of its cell.  convert_gaussian_xq (Sampler_impl.cuh:27-70) evaluates the same step function in float
-// arithmetic (trunc(3.2 * normcdfinvf(u / (2^32-1))), clamped to +-19.2); the two differ only for words within float rounding of a
-// step, and an integer rule is the same on every machine.
-struct GaussSteps {
-    uint32_t thr[19];
-};
-const GaussSteps& gauss_steps() {
-    static GaussSteps g = [] {
-        GaussSteps s;
-        for (int k = 1; k <= 19; k++) {
-            const double tail = 0.5 * std::erfc(((double)k / 3.2) / std::sqrt(2.0));
-            s.thr[k - 1] = (uint32_t)(4294967296.0 - std::floor(4294967296.0 * tail + 0.5));
-        }
-        return s;
-    }();
-    return g;
-}
-__device__ __forceinline__ int gauss_value(uint32_t u, const GaussSteps& g) {
-    int v = 0;
-#pragma unroll
-    for (int k = 0; k < 19; k++) {
-        v += (u >= g.thr[k]);
-        v -= (~u >= g.thr[k]);
-    }
-    return v;
-}
 __device__ __forceinline__ u64 signed_residue(int v, u64 q) { return v < 0 ? q + (long long)v : (u64)v; }
 __device__ __forceinline__ u64 zo_value(uint8_t byte, double t0, double t1, u64 q) {   // Sampler_impl.cuh:96-113
     const double d = (double)byte;
@@ -226,98 +212,129 @@ __global__ __launch_bounds__(THREADS) void encode_coeffs_kernel(u64* mx, const d
     mx[(long)t * N + i] = r < 0 ? (u64)(r + q) : (u64)r;
 }
 
-// Decoding table of one level (device words): w[i][j] = q_0..q_{j-1} mod q_i (row i, j < i), then cinv[i] = (q_0..q_{i-1})^-1 mod q_i,
-// then Q = q_0..q_l and floor(Q/2) as little-endian words.
+// Decoding table of one level: hatinv[i] = (Q/q_i)^-1 mod q_i and its Shoup word for each limb, then rows of COLS 30-bit words: Q/q_i for
+// each limb, 2^(30 COLS) - Q, Q, floor(Q/2).
 constexpr int DECODE_MAX_LIMBS = 64;
-
+constexpr int DECODE_AHEAD = 8;                                    // limbs whose words are requested together
+struct DecodeArgs {
+    double* vals;
+    const u64* coeff;
+    const PrimeConst* primes;                                      // of limb 0
+    const u64* tab;
+    long N;
+    int logN, limbs, fold_every, gap, is_bitrev;
+    double scale;
+};
+template <int COLS>
+__device__ __forceinline__ void carry30(u64 (&x)[COLS]) {          // columns -> 30-bit words, modulo 2^(30 COLS)
+    u64 c = 0;
+#pragma unroll
+    for (int k = 0; k < COLS; k++) {
+        c += x[k];
+        x[k] = c & 0x3fffffffu;
+        c >>= 30;
+    }
+}
 // CRT of one coefficient to the centred integer modulo Q, then to the nearest double, divided by the scale (Encoder.cuh:128-180,
-// NTL::ZZ there).  Garner's mixed-radix digits v_i (x = v_0 + v_1 q_0 + v_2 q_0 q_1 + ...) come first, Horner's rule over them gives x
-// as W machine words, x > floor(Q/2) is replaced by Q - x with a sign, and the top 64 significant bits plus a sticky bit round
-// correctly into the double.
-template <int W>
-__global__ __launch_bounds__(THREADS) void decode_coeffs_kernel(double* vals, const u64* coeff, const PrimeConst* primes, const u64* tab, long N, int logN,
-                                                                int K, int limbs, int gap, double scale, int is_bitrev) {
-    const long idx = (long)blockIdx.x * THREADS + threadIdx.x;
+// NTL::ZZ there):  x = sum_i y_i Q/q_i - v Q with y_i = x_i (Q/q_i)^-1 mod q_i and v = rint(sum_i y_i / q_i), which leaves x centred at
+// once.  The FP64 sum is within 2^-44 of the exact one, so v can only be one off where that sum lies within 2^-40 of a half; those
+// coefficients (about one in 2^39) are compared with floor(Q/2) word by word.  The products are summed in carry-free columns of 30 bits:
+// two multiply-adds per limb and column, one pass of carries at the end (and every fold_every limbs).
+// Bound by the latency of this chain: a ring has 256 .. 1024 waves, one per SIMD.  Mixed-radix digits (l^2/2 modular products that depend
+// on one another, then Horner's rule) in workgroups of 256 took 27.0 us for 10 limbs of 2^14, this 8.0: each wave is a workgroup of its
+// own, so that every compute unit takes part.
+template <int COLS>
+__global__ __launch_bounds__(64) void decode_coeffs_kernel(DecodeArgs a) {
+    const long idx = (long)blockIdx.x * 64 + threadIdx.x;
     long o = idx;
-    if (is_bitrev) o = (long)(__brev((uint32_t)idx) >> (32 - logN));
-    if (idx % gap) { vals[o] = 0.0; return; }                      // only coefficients j*gap and N/2 + j*gap are produced (:163-177)
-    const u64* wtab = tab;
-    const u64* cinv = tab + (long)limbs * limbs;
-    const u64* Qw = cinv + limbs;
-    const u64* Qh = Qw + W;
-    u64 v[DECODE_MAX_LIMBS];
-    v[0] = coeff[idx];
-    for (int i = 1; i < limbs; i++) {
-        const PrimeConst p = primes[K + i];
-        u64 acc = 0;
-        for (int j = 0; j < i; j++) {
-            u64 vj = v[j];
-            if (vj >= p.q) vj = barrett64(vj, p.q, p.mu_hi);
-            acc = csub(acc + mulmod(vj, wtab[(long)i * limbs + j], p), p.q);
-        }
-        const u64 diff = csub(p.q + coeff[(long)i * N + idx] - acc, p.q);
-        v[i] = mulmod(diff, cinv[i], p);
-    }
-    u64 x[W];
+    if (a.is_bitrev) o = (long)(__brev((uint32_t)idx) >> (32 - a.logN));
+    if (idx % a.gap) { a.vals[o] = 0.0; return; }                  // only coefficients j*gap and N/2 + j*gap are produced (:163-177)
+    const u64 *hatinv = a.tab, *hatinv_s = a.tab + a.limbs;
+    const unsigned* rows = (const unsigned*)(a.tab + 2 * a.limbs);
+    u64 x[COLS];
 #pragma unroll
-    for (int w = 0; w < W; w++) x[w] = 0;
-    x[0] = v[limbs - 1];
-    for (int i = limbs - 2; i >= 0; i--) {
-        const u64 q = primes[K + i].q;
-        u64 carry = v[i];
+    for (int k = 0; k < COLS; k++) x[k] = 0;
+    double s = 0.0;
+    int since = 0;
+    for (int i0 = 0; i0 < a.limbs; i0 += DECODE_AHEAD) {
+        u64 w[DECODE_AHEAD];
 #pragma unroll
-        for (int w = 0; w < W; w++) {
-            const u64 lo = x[w] * q, hi = __umul64hi(x[w], q);
-            const u64 sum = lo + carry;
-            carry = hi + (sum < lo);
-            x[w] = sum;
+        for (int i = 0; i < DECODE_AHEAD; i++) w[i] = a.coeff[(long)(i0 + i < a.limbs ? i0 + i : a.limbs - 1) * a.N + idx];
+#pragma unroll
+        for (int i = 0; i < DECODE_AHEAD; i++) {
+            if (i0 + i >= a.limbs) break;
+            const int l = i0 + i;
+            const u64 y = mul_shoup(w[i], hatinv[l], hatinv_s[l], a.primes[l].q);
+            s = __builtin_fma((double)y, a.primes[l].qinv_d, s);
+            const unsigned y0 = (unsigned)y & 0x3fffffffu, y1 = (unsigned)(y >> 30);
+            const unsigned* row = rows + (long)l * COLS;
+            x[0] += (u64)y0 * row[0];
+#pragma unroll
+            for (int k = 1; k < COLS; k++) x[k] += (u64)y0 * row[k] + (u64)y1 * row[k - 1];
+            if (++since == a.fold_every) { carry30<COLS>(x); since = 0; }
         }
     }
-    // x > floor(Q/2) ?
-    bool greater = false, decided = false;
+    const double v = __builtin_rint(s);
+    const unsigned* neg_q = rows + (long)a.limbs * COLS;
 #pragma unroll
-    for (int w = W - 1; w >= 0; w--) {
-        const u64 h = Qh[w];
-        if (!decided && x[w] != h) { greater = x[w] > h; decided = true; }
-    }
-    if (greater) {
-        u64 borrow = 0;
+    for (int k = 0; k < COLS; k++) x[k] += (u64)(unsigned)v * neg_q[k];
+    carry30<COLS>(x);
+    bool negative = (x[COLS - 1] >> 29) != 0;
+    if (negative) {
+        u64 c = 1;
 #pragma unroll
-        for (int w = 0; w < W; w++) {
-            const u64 qv = Qw[w];
-            const u64 d1 = qv - x[w];
-            const u64 b1 = qv < x[w];
-            const u64 d2 = d1 - borrow;
-            const u64 b2 = d1 < borrow;
-            x[w] = d2;
-            borrow = b1 | b2;
+        for (int k = 0; k < COLS; k++) {
+            c += x[k] ^ 0x3fffffffu;
+            x[k] = c & 0x3fffffffu;
+            c >>= 30;
         }
     }
-    // top word, the word below it, sticky bits
-    u64 top = 0, next = 0;
+    if (__builtin_fabs(s - v) > 0.5 - 9.094947017729282e-13) {
+        const unsigned *qw = neg_q + COLS, *half = qw + COLS;
+        bool greater = false;
+#pragma unroll
+        for (int k = 0; k < COLS; k++) greater = x[k] == half[k] ? greater : x[k] > half[k];
+        if (greater) {                                             // v was one off: Q - |x| with the other sign
+            u64 c = 1;
+#pragma unroll
+            for (int k = 0; k < COLS; k++) {
+                c += (x[k] ^ 0x3fffffffu) + qw[k];
+                x[k] = c & 0x3fffffffu;
+                c >>= 30;
+            }
+            negative = !negative;
+        }
+    }
+    // the three words from the top one down, sticky bits below them
+    unsigned top = 0, mid = 0, low = 0;
     bool sticky = false;
-    int k = 0;
-    bool found = false;
+    int at = 0;
 #pragma unroll
-    for (int w = W - 1; w >= 0; w--) {
-        if (!found) {
-            if (x[w] != 0) { found = true; top = x[w]; k = w; next = w > 0 ? x[w - 1] : 0; }
-        } else if (w < k - 1) {
-            sticky = sticky || x[w] != 0;
+    for (int k = COLS - 1; k >= 0; k--) {
+        const unsigned w = (unsigned)x[k];
+        if (top == 0) {
+            if (w) { top = w; at = k; mid = k > 0 ? (unsigned)x[k > 0 ? k - 1 : 0] : 0; low = k > 1 ? (unsigned)x[k > 1 ? k - 2 : 0] : 0; }
+        } else if (k < at - 2) {
+            sticky = sticky || w != 0;
         }
     }
     double d = 0.0;
-    if (found) {
-        const int lz = __clzll((long long)top);
-        u64 m = top << lz;
-        if (lz) { m |= next >> (64 - lz); sticky = sticky || (next << lz) != 0; } else { sticky = sticky || next != 0; }
+    if (top) {
+        const int n = 32 - __clz((int)top);                        // 1 .. 30: the three words hold 60 + n bits
+        u64 m = ((u64)top << (64 - n)) | ((u64)mid << (34 - n));
+        if (n >= 4) {
+            m |= low >> (n - 4);
+            sticky = sticky || (low & ((1u << (n - 4)) - 1u)) != 0;
+        } else {
+            m |= (u64)low << (4 - n);
+        }
         if (sticky) m |= 1;
-        d = ldexp(__ull2double_rn(m), 64 * k - lz);
-        if (greater) d = -d;
+        d = ldexp(__ull2double_rn(m), 30 * (at - 2) + n - 4);
+        if (negative) d = -d;
     }
-    d /= scale;
-    if (is_bitrev) d *= 256;                                       // Encoder.cuh:171-173
-    vals[o] = d;
+    d /= a.scale;
+    if (a.is_bitrev) d *= 256;                                     // Encoder.cuh:171-173
+    a.vals[o] = d;
 }
 
 int check_limbs(ckks_ctx* c, const void* a, const void* b, int idx_out, int idx_mod, int mod_num, const char* who) {
@@ -467,6 +484,8 @@ extern "C" int ckks_encrypt(ckks_ctx* c, uint64_t* cipher, const uint64_t* mx, c
     if (rc != CKKS_OK) return rc;
     if (!cipher || !pk || !random || !scratch) { set_error("encryptMsg: null argument"); return CKKS_E_INVALID; }
     if (((uintptr_t)random) & 3) { set_error("encryptMsg: random words must be 4-byte aligned"); return CKKS_E_INVALID; }
+    bool done = false;
+    if ((rc = launch_encrypt_lines(c, cipher, mx, pk, random, scratch, l, &done)) || done) return rc;
     const int K = c->K, L1 = c->L + 1;
     const long N = c->N;
     u64* ax = (u64*)cipher;
@@ -500,43 +519,71 @@ extern "C" int ckks_encode_coeffs(ckks_ctx* c, uint64_t* mx, const double* vals,
     int rc = check_level(c, l, "encode_coeffs");
     if (rc != CKKS_OK) return rc;
     if (!mx || !vals) { set_error("encode_coeffs: null argument"); return CKKS_E_INVALID; }
+    bool done = false;
+    if ((rc = launch_encode_lines(c, mx, vals, scale, l, &done)) || done) return rc;
     const long N = c->N;
     hipLaunchKernelGGL(encode_coeffs_kernel, dim3(N / THREADS, l + 1), dim3(THREADS), 0, c->stream, (u64*)mx, vals, c->d_primes, N, c->K, scale);
     CKKS_HIP_TRY(hipGetLastError());
     return launch_ntt(c, mx, 0, c->K, 1, l + 1, c->L + 1, 0, 1, false);
 }
 
+// columns of the kernel that takes a modulus of so many bits (one bit for the sign, one to spare); 0: none does
+static int decode_cols(int bits) {
+    for (int cols : {4, 9, 18, 35, 69})
+        if (30 * cols >= bits + 2) return cols;
+    return 0;
+}
+static int bit_length(const std::vector<u64>& x) {
+    for (size_t w = x.size(); w-- > 0;)
+        if (x[w]) return (int)(64 * w) + 64 - __builtin_clzll(x[w]);
+    return 0;
+}
+static void words30(const std::vector<u64>& x, int cols, unsigned* out) {
+    for (int k = 0; k < cols; k++) {
+        const size_t bit = (size_t)30 * k, w = bit / 64, r = bit % 64;
+        u64 v = w < x.size() ? x[w] >> r : 0;
+        if (r > 34 && w + 1 < x.size()) v |= x[w + 1] << (64 - r);
+        out[k] = (unsigned)v & 0x3fffffffu;
+    }
+}
+
 // table of one level, built on first use and kept until the context is destroyed
-static int decode_table(ckks_ctx* c, int l, const u64** tab, int* words) {
+static int decode_table(ckks_ctx* c, int l, const u64** tab, int* cols_out) {
     for (auto& e : c->decode_tabs)
-        if (e.level == l) { *tab = (const u64*)e.dev; *words = e.words; return CKKS_OK; }
+        if (e.level == l) { *tab = (const u64*)e.dev; *cols_out = e.words; return CKKS_OK; }
     const int n = l + 1;
     const u64* q = c->pqt.data() + c->K;
     std::vector<u64> Q{1};
     for (int i = 0; i < n; i++) big_mul_word(Q, q[i]);
-    int W = 8;
-    while (W < (int)Q.size()) W *= 2;
-    if (W > 32) { set_error("decode_coeffs: modulus above 2048 bits"); return CKKS_E_INVALID; }
-    std::vector<u64> host((size_t)n * n + n + 2 * W, 0);
+    const int cols = bit_length(Q) > 2048 ? 0 : decode_cols(bit_length(Q));
+    if (!cols) { set_error("decode_coeffs: modulus above 2048 bits"); return CKKS_E_INVALID; }
+    std::vector<u64> host((size_t)2 * n + ((size_t)(n + 3) * cols + 1) / 2, 0);
+    unsigned* rows = (unsigned*)(host.data() + 2 * n);
     for (int i = 0; i < n; i++) {
+        std::vector<u64> hat{1};
         u64 prod = 1 % q[i];
-        for (int j = 0; j < i; j++) {
-            host[(size_t)i * n + j] = prod;
-            prod = H::mulmod(prod, q[j] % q[i], q[i]);
-        }
-        host[(size_t)n * n + i] = i ? H::invmod(prod, q[i]) : 1;
+        for (int j = 0; j < n; j++)
+            if (j != i) { big_mul_word(hat, q[j]); prod = H::mulmod(prod, q[j] % q[i], q[i]); }
+        host[i] = n > 1 ? H::invmod(prod, q[i]) : 1 % q[i];
+        host[n + i] = H::shoup(host[i], q[i]);
+        words30(hat, cols, rows + (size_t)i * cols);
     }
-    u64* Qw = host.data() + (size_t)n * n + n;
-    u64* Qh = Qw + W;
-    for (size_t w = 0; w < Q.size(); w++) Qw[w] = Q[w];
-    for (int w = 0; w < W; w++) Qh[w] = (Qw[w] >> 1) | (w + 1 < W ? Qw[w + 1] << 63 : 0);
+    unsigned *neg_q = rows + (size_t)n * cols, *qw = neg_q + cols, *half = qw + cols;
+    words30(Q, cols, qw);
+    u64 carry = 1;
+    for (int k = 0; k < cols; k++) {
+        carry += qw[k] ^ 0x3fffffffu;
+        neg_q[k] = (unsigned)carry & 0x3fffffffu;
+        carry >>= 30;
+        half[k] = (qw[k] >> 1) | (k + 1 < cols ? (qw[k + 1] & 1u) << 29 : 0u);
+    }
     void* dev = nullptr;
     CKKS_HIP_TRY(hipMalloc(&dev, host.size() * 8));
     hipError_t e = hipMemcpy(dev, host.data(), host.size() * 8, hipMemcpyHostToDevice);
     if (e != hipSuccess) { (void)hipFree(dev); return hip_fail(e, "hipMemcpy(decode table)"); }
-    c->decode_tabs.push_back({l, W, dev});
+    c->decode_tabs.push_back({l, cols, dev});
     *tab = (const u64*)dev;
-    *words = W;
+    *cols_out = cols;
     return CKKS_OK;
 }
 
@@ -549,21 +596,29 @@ extern "C" int ckks_decode_coeffs(ckks_ctx* c, double* vals, const uint64_t* mx,
     if (l + 1 > DECODE_MAX_LIMBS) { set_error("decode_coeffs: more than 64 limbs"); return CKKS_E_INVALID; }
     if (!(scale > 0)) { set_error("decode_coeffs: scale must be positive"); return CKKS_E_INVALID; }
     const u64* tab = nullptr;
-    int W = 0;
-    rc = decode_table(c, l, &tab, &W);
+    int cols = 0;
+    rc = decode_table(c, l, &tab, &cols);
     if (rc != CKKS_OK) return rc;
-    CKKS_HIP_TRY(hipMemcpyAsync(scratch, mx, 8 * N * (size_t)(l + 1), hipMemcpyDeviceToDevice, c->stream));
-    rc = launch_ntt(c, scratch, 0, c->K, 1, l + 1, l + 1, 0, 1, true);
-    if (rc != CKKS_OK) return rc;
-    const int gap = (int)((N / 2) / slots);
-    dim3 grid((unsigned)(N / THREADS)), block(THREADS);
-#define LAUNCH_DECODE(WW)                                                                                                              \
-    hipLaunchKernelGGL(decode_coeffs_kernel<WW>, grid, block, 0, c->stream, vals, (const u64*)scratch, c->d_primes, tab, N, c->logN, c->K, l + 1, gap, \
-                       scale, is_bitrev)
-    if (W == 8) LAUNCH_DECODE(8);
-    else if (W == 16) LAUNCH_DECODE(16);
-    else LAUNCH_DECODE(32);
-#undef LAUNCH_DECODE
+    bool done = false;
+    if ((rc = launch_coefficients_lines(c, scratch, mx, l, &done))) return rc;
+    if (!done) {
+        CKKS_HIP_TRY(hipMemcpyAsync(scratch, mx, 8 * N * (size_t)(l + 1), hipMemcpyDeviceToDevice, c->stream));
+        if ((rc = launch_ntt(c, scratch, 0, c->K, 1, l + 1, l + 1, 0, 1, true))) return rc;
+    }
+    u64 most = 0;
+    for (int i = 0; i <= l; i++) most = std::max<u64>(most, c->pqt[c->K + i]);
+    DecodeArgs d;
+    d.vals = vals; d.coeff = (const u64*)scratch; d.primes = c->d_primes + c->K; d.tab = tab; d.N = N; d.logN = c->logN; d.limbs = l + 1;
+    d.fold_every = (int)((15ull << 30) / ((1ull << 30) + (most >> 30) + 1));      // a limb adds less than 2^60 + 2^30 (q / 2^30 + 1) to a column
+    d.gap = (int)((N / 2) / slots); d.is_bitrev = is_bitrev; d.scale = scale;
+    const dim3 grid((unsigned)(N / 64)), block(64);
+    switch (cols) {
+        case 4: hipLaunchKernelGGL(decode_coeffs_kernel<4>, grid, block, 0, c->stream, d); break;
+        case 9: hipLaunchKernelGGL(decode_coeffs_kernel<9>, grid, block, 0, c->stream, d); break;
+        case 18: hipLaunchKernelGGL(decode_coeffs_kernel<18>, grid, block, 0, c->stream, d); break;
+        case 35: hipLaunchKernelGGL(decode_coeffs_kernel<35>, grid, block, 0, c->stream, d); break;
+        default: hipLaunchKernelGGL(decode_coeffs_kernel<69>, grid, block, 0, c->stream, d);
+    }
     CKKS_HIP_TRY(hipGetLastError());
     return CKKS_OK;
 }

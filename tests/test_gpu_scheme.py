@@ -1,12 +1,15 @@
 """GPU parity of the client-side entry points (random stream, samplers, pointwise arithmetic, keys, encryption, decryption,
 coefficient encode / decode) through the C ABI against the CPU oracle: bit-exact on every integer word; the decoder's doubles
 exact for power-of-two scales and within one unit in the last place otherwise."""
+import math
+
 import numpy as np
 import pytest
 
 from ckks_llm_amd import CkksError, Ciphertext, Context_23, DeviceBuffer, Plaintext, Scheme_23, SecretKey
 from oracle import oracle_py as O
 from tests.gpu_common import Pair, to_dev, from_dev
+from ckks_llm_amd.params import REF_PARAMS
 from tests.params import CFG2_Q, CFG3_P
 
 pytestmark = pytest.mark.gpu
@@ -232,6 +235,63 @@ def test_decoder_rounds_to_nearest_with_sticky_bits():
     got = d_out.download(np.float64)
     assert [float(c) for c in cs[:10]] == list(got[:10])                 # Python's int -> float is correctly rounded
     assert not got[10:].any()
+
+
+@pytest.mark.parametrize("logN,bits,nq", [(12, 36, 1), (12, 49, 5), (13, 36, 9), (14, 49, 3), (15, 36, 2), (15, 49, 12)])
+def test_steps_inside_the_transforms_match_separate_steps(logN, bits, nq):
+    """encode, encrypt (with and without a message) and decode in line transforms against the separate steps (option ks_split), bit
+    for bit, at the lowest and the highest level; values whose product with the scale needs all 64 bits among them."""
+    q = (CFG2_Q if bits == 36 else REF_PARAMS[16]["q"])[:nq]
+    dev = Context_23(logN, CFG3_P[:1], q)
+    N, L_ = dev.N, dev.L_
+    rng = np.random.default_rng(logN * nq)
+    vals = rng.normal(0, 2.0, N)
+    vals[:6] = [0.0, -0.0, 2.0 ** 22, -(2.0 ** 23), 2.0 ** -41, -1.0 + 2.0 ** -40]
+    d_vals, rnd = DeviceBuffer.from_numpy(vals), dev_bytes(rng.integers(0, 256, 9 * N, dtype=np.uint8))
+    pk = to_dev(np.stack([[rng.integers(0, m, N, dtype=np.uint64) for m in q] for _ in range(2)]))
+    scratch = DeviceBuffer(8 * N * nq)
+    for l in sorted({0, nq - 1}):
+        got = {}
+        for split in (1, 0):
+            dev.set_option("ks_split", split)
+            mx, ct, ct0 = (to_dev(np.full((k, nq, N), 3, dtype=np.uint64)) for k in (1, 2, 2))
+            out = DeviceBuffer(8 * N)
+            assert L_.ckks_encode_coeffs(dev.h, mx.ptr, d_vals.ptr, 1 << 40, l) == 0
+            assert L_.ckks_encrypt(dev.h, ct.ptr, mx.ptr, pk.ptr, rnd.ptr, scratch.ptr, l) == 0
+            assert L_.ckks_encrypt(dev.h, ct0.ptr, None, pk.ptr, rnd.ptr, scratch.ptr, l) == 0
+            assert L_.ckks_decode_coeffs(dev.h, out.ptr, mx.ptr, scratch.ptr, float(1 << 40), N // 2, 0, l) == 0
+            got[split] = [b.download() for b in (mx, ct, ct0, out)]
+        for a, b in zip(got[0], got[1]):
+            assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("bits,nq", [(36, 1), (36, 3), (49, 5), (60, 7), (60, 8), (49, 21), (36, 24), (49, 28)])
+def test_decoder_at_the_ends_of_the_range(bits, nq):
+    """Integers at and beside 0, +-Q/2 and the powers of two where the decoder's words end, through every word count that it is built
+    for and both of its carry intervals: the nearest doubles."""
+    q = {36: CFG2_Q, 49: REF_PARAMS[16]["q"], 60: REF_PARAMS[16]["t"]}[bits][:nq]
+    pair = Pair(8, CFG3_P[:1], q)
+    N, Q = pair.N, 1
+    for m in q:
+        Q *= m
+    h = Q // 2
+    cs = [0, 1, -1, h, -h, h - 1, 1 - h, h - (h >> 41), (h >> 41) - h]
+    for k in range(30, h.bit_length() - 1, 30):
+        cs += [1 << k, (1 << k) - 1, -(1 << k), 1 - (1 << k)]
+    rng = np.random.default_rng(nq)
+    while len(cs) < N:
+        cs.append((int.from_bytes(rng.bytes(256), "little") % Q - h) >> int(rng.integers(0, h.bit_length())))
+    res = np.array([[c % m for c in cs] for m in q], dtype=np.uint64)
+    pair.orc.ToNTTInplace(res.reshape(-1), 0, 1, 1, nq, nq)
+    out, scratch = DeviceBuffer(8 * N), DeviceBuffer(8 * N * nq)
+    assert pair.dev.L_.ckks_decode_coeffs(pair.dev.h, out.ptr, to_dev(res).ptr, scratch.ptr, 1.0, N // 2, 0, nq - 1) == 0
+
+    def nearest(c):
+        try:
+            return float(c)
+        except OverflowError:                                             # beyond the largest double
+            return math.inf if c > 0 else -math.inf
+    assert [nearest(c) for c in cs] == list(out.download(np.float64))
 
 
 def test_mirror_classes_encrypt_decrypt_decode():
