@@ -239,44 +239,6 @@ __global__ __launch_bounds__(256) void ppmm_generic_kernel(PpmmArgs a) {
     }
 }
 
-// ------------------------------------------------------------------------------------------------------------
-// Plaintext matrices wider than one MFMA launch takes (more than 4 balanced digits, 3 with the 7-digit residues) are cut into
-// slices of three digits, A = sum_s A_s 2^(24 s): one launch per slice writes the residues of A_s x Ct as they are, and this
-// kernel forms sum_s (2^(24 s) mod q) * slice_s mod q and then the fused rescale of PPMM_kernel.cuh:213-249 - the same
-// integers as one pass over the whole of A, since every step is exact modulo the prime.
-// ------------------------------------------------------------------------------------------------------------
-struct PpmmCombineArgs {
-    u64* out;                     // slice 0 on entry, the result on return; [M][mod_num][C]
-    const u64* more;              // slices 1 .. slices-1, each [M][mod_num][C]
-    const PrimeConst* pq;
-    const u64* consts;            // row 0: q_last^-1 mod q_i, row 1: its Shoup word
-    long C, per_slice;            // per_slice = M * mod_num * C
-    int M, mod_num, np, slices;
-    u64 w[2][PPMM_MAX_MODS];      // 2^24 mod q_i, 2^48 mod q_i
-};
-__global__ __launch_bounds__(256) void ppmm_combine_kernel(PpmmCombineArgs a) {
-    const long c = (long)blockIdx.x * 256 + threadIdx.x;
-    const int m = blockIdx.y;
-    if (c >= a.C) return;
-    u64* o = a.out + (long)m * a.C * a.mod_num;
-    const u64* t = a.more + (long)m * a.C * a.mod_num;
-    u64 r_last = 0;
-    for (int im = a.mod_num - 1; im >= 0; im--) {
-        const PrimeConst& pr = a.pq[a.np + im];
-        const long idx = (long)im * a.C + c;
-        u128w acc = {o[idx], 0};
-        for (int s = 1; s < a.slices; s++) mac128(acc, t[(long)(s - 1) * a.per_slice + idx], a.w[s - 1][im]);
-        const u64 r = barrett128(acc, pr.q, pr.mu_hi, pr.mu_lo);
-        if (im == a.mod_num - 1) {
-            r_last = r;
-            o[idx] = r;
-        } else {
-            const u64 temp = r + pr.q - r_last;                             // PPMM_kernel.cuh:244
-            o[idx] = mul_shoup(temp, a.consts[im], a.consts[PPMM_MAX_MODS + im], pr.q);
-        }
-    }
-}
-
 }  // namespace ckks
 
 using namespace ckks;
@@ -315,7 +277,7 @@ extern "C" int pcmm_ctx_destroy(pcmm_ctx* h) {
     if (!h) return CKKS_OK;
     { std::lock_guard<std::mutex> lock(g_handles_mutex); g_handles.erase(std::remove(g_handles.begin(), g_handles.end(), h), g_handles.end()); }
     (void)hipDeviceSynchronize();
-    void* ptrs[] = {h->d_pq, h->d_ptrs, h->d_absmax, h->d_zero, h->d_Bdig, h->d_small_tw, h->d_slices, h->d_workA, h->d_workAdig};
+    void* ptrs[] = {h->d_pq, h->d_ptrs, h->d_absmax, h->d_zero, h->d_Bdig, h->d_small_tw, h->d_workA, h->d_workAdig};
     for (void* p : ptrs) if (p) (void)hipFree(p);
     for (auto& w : h->weights) { if (w.d_A) (void)hipFree(w.d_A); if (w.d_Adig) (void)hipFree(w.d_Adig); }
     if (h->pin) (void)hipHostFree(h->pin);
@@ -757,6 +719,7 @@ static int ppmm_common(pcmm_ctx* h, const float* W, const uint64_t* const* ptrs_
             }
             cst[2 * PPMM_MAX_MODS + i] = dbits(H::powmod(2, 32, qi), qi);
             cst[3 * PPMM_MAX_MODS + i] = dbits(H::powmod(2, 64, qi), qi);
+            cst[5 * PPMM_MAX_MODS + i] = dbits(H::powmod(2, 24, qi), qi);
         }
         if ((rc = stage_to_device(h, d_cst, cst.data(), PPMM_CONST_WORDS * sizeof(uint64_t)))) return rc;
         h->cst_mods = mod_num;
@@ -897,30 +860,19 @@ static int ppmm_common(pcmm_ctx* h, const float* W, const uint64_t* const* ptrs_
             rc = launch_ppmm_mfma_impl(c->stream, a, DW, DC, h->d_Bdig, !packed && !packed_early);
             if (rc) return rc;
         } else {
-            const size_t per_slice = (size_t)M * mod_num * C;
-            if ((slices - 1) * per_slice > h->slices_cap) {
-                if (h->d_slices) { (void)hipDeviceSynchronize(); (void)hipFree(h->d_slices); h->d_slices = nullptr; h->slices_cap = 0; }
-                hipError_t e = hipMalloc((void**)&h->d_slices, (slices - 1) * per_slice * sizeof(uint64_t));
-                if (e != hipSuccess) { set_error("PPMM: cannot allocate the buffers of the plaintext slices"); return CKKS_E_NOMEM; }
-                h->slices_cap = (slices - 1) * per_slice;
-            }
+            // Plaintext matrices wider than one launch takes (more than 4 balanced digits, 3 with the 7-digit residues) go in slices of three digits,
+            // A = sum_s A_s 2^(24 s), from the top one down: each leaves its residues in the output, the next adds them times 2^24 to its own, and
+            // the lowest applies the fused rescale of PPMM_kernel.cuh:213-249 - the same integers as one pass over the whole of A, since every
+            // step is exact modulo the prime.  Slices kept side by side and combined by a pass of their own, at copy speed over 2.4 GB, took 517 us
+            // at 768 x 768 over two 49-bit moduli and a buffer per slice; the carry costs the lower slice 220 us (1616 for 1399, of which 0.8 GB take 170).
             PpmmArgs sa = a;
-            sa.raw_all = 1;
-            for (int sl = 0; sl < slices; sl++) {
+            for (int sl = slices - 1; sl >= 0; sl--) {
                 sa.Adig = we->d_Adig + (size_t)3 * sl * Mpad * Kpad;
-                sa.out = sl == 0 ? out : h->d_slices + (size_t)(sl - 1) * per_slice;
-                rc = launch_ppmm_mfma_impl(c->stream, sa, 3, DC, h->d_Bdig, !packed && !packed_early && sl == 0);      // the residue planes are packed once
+                sa.raw_all = sl > 0;
+                sa.carry = sl < slices - 1;
+                rc = launch_ppmm_mfma_impl(c->stream, sa, 3, DC, h->d_Bdig, !packed && !packed_early && sl == slices - 1);      // the residue planes are packed once
                 if (rc) return rc;
             }
-            PpmmCombineArgs ca;
-            ca.out = out; ca.more = h->d_slices; ca.pq = h->d_pq; ca.consts = d_cst; ca.C = C; ca.per_slice = (long)per_slice;
-            ca.M = M; ca.mod_num = mod_num; ca.np = h->np; ca.slices = slices;
-            for (int i = 0; i < mod_num; i++) {
-                const uint64_t qi = h->pq[h->np + i];
-                ca.w[0][i] = H::powmod(2, 24, qi);
-                ca.w[1][i] = H::powmod(2, 48, qi);
-            }
-            hipLaunchKernelGGL(ppmm_combine_kernel, dim3((unsigned)((C + 255) / 256), M), dim3(256), 0, c->stream, ca);
         }
     } else {
         dim3 grid((unsigned)((C + 255) / 256), M), block(256);

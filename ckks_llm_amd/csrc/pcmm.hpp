@@ -19,8 +19,6 @@ struct pcmm_ctx {
     int packed_K = 0, packed_mods = 0;       // shape the residue digit planes were opened for by pcmm_packed_begin (0: not open)
     int last_path = -1, last_DW = 0, last_DC = 0;   // what the last PPMM call ran: 1 = MFMA kernel, 0 = generic kernel
     int last_slices = 0;                     // plaintext digit slices of the last MFMA call (1: one launch with the fused rescale)
-    uint64_t* d_slices = nullptr;            // outputs of the plaintext slices above the first, [slice - 1][M][mod_num][C]
-    size_t slices_cap = 0;
     unsigned long long last_absmax = 0;
     ckks_ctx* small = nullptr;               // tables of the size-N1 transform over the ring-pack primes, built on first use
     uint64_t* d_small_tw = nullptr;          // tables of the size-N1 transform when N1 < 256: [prime][forward | inverse][N1]
@@ -69,9 +67,10 @@ namespace ckks {
 
 // per-call constants of the PPMM epilogue, one row of PPMM_MAX_MODS words each:
 //   [0] q_last^-1 mod q_i   [1] its Shoup word   [2] 2^32 mod q_i   [3] 2^64 mod q_i   [4] q_last^-1 mod q_i
-//   rows 2..4 are balanced representatives stored as IEEE double bit patterns (FP64 epilogue)
+//   [5] 2^24 mod q_i
+//   rows 2..5 are balanced representatives stored as IEEE double bit patterns (FP64 epilogue)
 constexpr int PPMM_MAX_MODS = 64;
-constexpr int PPMM_CONST_ROWS = 5;
+constexpr int PPMM_CONST_ROWS = 6;
 constexpr int PPMM_CONST_WORDS = PPMM_MAX_MODS * PPMM_CONST_ROWS;
 
 struct PpmmArgs {
@@ -85,7 +84,8 @@ struct PpmmArgs {
     const u64* consts;            // PPMM_CONST_WORDS words, see above
     long C;
     int M, Kin, Mpad, Kpad, mod_num, np;
-    int raw_all;                  // MFMA kernel: store every modulus' residue as it is (no fused rescale); the caller combines slices
+    int raw_all;                  // MFMA kernel: store every modulus' residue as it is (no fused rescale): a slice above the lowest
+    int carry = 0;                // MFMA kernel: add 2^24 times what the output holds (the slice above; a three-digit slice)
     int no_tail = 0;              // MFMA kernel: run the remainder column panels whole instead of as jobs by prime (tuning switch)
 };
 

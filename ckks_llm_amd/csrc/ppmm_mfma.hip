@@ -110,7 +110,10 @@ __global__ __launch_bounds__(256) void ppmm_pack_kernel(PpmmArgs a, int8_t* __re
 //   NWAVES = 8, RING = 3: 128 x 64 tile, one workgroup per CU (135 KiB of LDS), loads issued two steps ahead.
 // The other shape that fits the LDS (NWAVES = 4, RING = 2: 64 x 64 tile, 64 KiB, two workgroups per CU that drift out of phase)
 // was measured and is no faster (its single step of load lead time costs what the overlap of the two workgroups gains).
-template <int DW, int NWAVES, int RING, int DC>
+// CARRY: a lower slice of a plaintext matrix of several (A = sum_s A_s 2^(24 s), three digits each): the residues that the slice above it has left in
+// the output, times 2^24, are added to this slice's before they are reduced (Horner's rule over the slices, from the top one down).  A
+// lane reads the words that it then writes.
+template <int DW, int NWAVES, int RING, int DC, bool CARRY>
 __global__ __launch_bounds__(64 * NWAVES, 2) void ppmm_mfma_kernel(PpmmArgs a, const int8_t* __restrict__ bdig, int c_tiles, int m_block,
                                                                    int main_blocks, int tail_jobs) {
     constexpr int ND = DW + DC - 1, MT = 16 * NWAVES;
@@ -289,7 +292,7 @@ __global__ __launch_bounds__(64 * NWAVES, 2) void ppmm_mfma_kernel(PpmmArgs a, c
     unsigned rl_lo[2][4][2], rl_hi[2][2];
     double rl_wide[WIDE ? 2 : 1][WIDE ? 2 : 1][WIDE ? 4 : 1];           // the wide form keeps r_last as doubles
     // constants of the prime in work, requested before its K loop so that the epilogue does not start with a round trip to memory
-    double q = 0, qinv = 0, c32 = 0, c64 = 0, qli = 0;
+    double q = 0, qinv = 0, c24 = 0, c32 = 0, c64 = 0, qli = 0;
     auto epilogue = [&](int im, auto last_c, auto full_c) {
         constexpr bool LAST = decltype(last_c)::value, FULL = decltype(full_c)::value;
         // The output addressing starts from a value the optimiser cannot hoist above the K loop (it would otherwise keep
@@ -301,6 +304,17 @@ __global__ __launch_bounds__(64 * NWAVES, 2) void ppmm_mfma_kernel(PpmmArgs a, c
         int mrow = m0 + wm * 32 + 4 * lg;
         asm volatile("" : "+v"(mrow));
         u64* obase = a.out + (long)im * a.C + c0 + wc * 32 + lr;
+        // the carried words of an MFMA tile, requested a tile ahead and so ahead of the stores of the tile before, which a wait for them would
+        // include: 1616 us per launch at 768 x 768 over two 49-bit moduli, 1697 with each tile's words requested at its own start
+        u64 above[2][4] = {};
+        auto fetch = [&](int tile, u64 (&dst)[4]) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int row = mrow + (tile >> 1) * 16 + r;
+                dst[r] = obase[(long)(FULL || row < a.M ? row : a.M - 1) * row_stride + (tile & 1) * 16];
+            }
+        };
+        if constexpr (CARRY) fetch(0, above[0]);
 #pragma unroll
         for (int mt = 0; mt < 2; mt++) {
             // rows of the M padding are clamped for addressing; their stores are skipped
@@ -312,6 +326,9 @@ __global__ __launch_bounds__(64 * NWAVES, 2) void ppmm_mfma_kernel(PpmmArgs a, c
             }
 #pragma unroll
             for (int nt = 0; nt < 2; nt++) {
+                if constexpr (CARRY) {
+                    if (2 * mt + nt < 3) fetch(2 * mt + nt + 1, above[(nt + 1) & 1]);
+                }
                 if constexpr (WIDE) {
                     // q < 2^50.  Groups of four diagonals y0 (e < 4), y1 (4 <= e < 8), y2 (e >= 8), each exact below 2^53; y0 and y1
                     // are first brought to (-q/2, q/2] so that the products with 2^32 and 2^64 mod q stay below 2^99 (quotients below
@@ -341,7 +358,11 @@ __global__ __launch_bounds__(64 * NWAVES, 2) void ppmm_mfma_kernel(PpmmArgs a, c
 #pragma unroll
                     for (int r = 0; r < 4; r++) y2[r] = mulmod_f64(y2[r], c64, q, qinv);
 #pragma unroll
-                    for (int r = 0; r < 4; r++) t[r] = balance_f64(y0[r] + y1[r] + y2[r], q, qinv);
+                    for (int r = 0; r < 4; r++) {
+                        t[r] = y0[r] + y1[r] + y2[r];
+                        if constexpr (CARRY) t[r] += mulmod_f64(exact_u2d(above[nt & 1][r]), c24, q, qinv);     // four terms within 0.51 q
+                        t[r] = balance_f64(t[r], q, qinv);
+                    }
                     if (!LAST) {
 #pragma unroll
                         for (int r = 0; r < 4; r++) t[r] = balance_f64(mulmod_f64(t[r] - rl_wide[WIDE ? mt : 0][WIDE ? nt : 0][WIDE ? r : 0], qli, q, qinv), q, qinv);
@@ -384,6 +405,10 @@ __global__ __launch_bounds__(64 * NWAVES, 2) void ppmm_mfma_kernel(PpmmArgs a, c
                     for (int r = 0; r < 4; r++) c[r] = __builtin_rint(h[r] * qinv);
 #pragma unroll
                     for (int r = 0; r < 4; r++) t[r] = y0[r] + (__builtin_fma(-c[r], q, h[r]) + l[r]);
+                    if constexpr (CARRY) {                               // another 0.51 q < 2^38: |y0| is below 2^52.1, the sum stays exact
+#pragma unroll
+                        for (int r = 0; r < 4; r++) t[r] += mulmod_f64(exact_u2d(above[nt & 1][r]), c24, q, qinv);
+                    }
 #pragma unroll
                     for (int r = 0; r < 4; r++) c[r] = __builtin_rint(t[r] * qinv);
 #pragma unroll
@@ -432,6 +457,7 @@ __global__ __launch_bounds__(64 * NWAVES, 2) void ppmm_mfma_kernel(PpmmArgs a, c
         const int im = prime_of(it);
         q = a.pq[a.np + im].qd;
         qinv = a.pq[a.np + im].qinv_d;
+        if (CARRY) c24 = f64_from_bits(a.consts[5 * PPMM_MAX_MODS + im]);  // 2^24 mod q (balanced)
         c32 = f64_from_bits(a.consts[2 * PPMM_MAX_MODS + im]);   // 2^32 mod q (balanced)
         if (WIDE) c64 = f64_from_bits(a.consts[3 * PPMM_MAX_MODS + im]);   // 2^64 mod q (balanced)
         qli = f64_from_bits(a.consts[4 * PPMM_MAX_MODS + im]);   // q_last^-1 mod q
@@ -471,16 +497,22 @@ static int launch_dw(hipStream_t stream, const PpmmArgs& a, int8_t* bdig, bool p
     for (int d = 2; d <= 8; d++) if (m_tiles % d == 0) m_block = d;
     unsigned blocks = (unsigned)((c_tiles + 7) / 8) * 8u * (unsigned)m_tiles;
     // The column panels beyond the last full group of eight (one per XCD) are cut into jobs by prime where that pays: a single patch
-    // of row tiles (small M), enough primes to share, and the fused rescale (a job needs the last prime only then).
+    // of row tiles (small M), enough primes to share, and the fused rescale (a job needs the last prime only then) of a whole matrix (the jobs
+    // of a tile all form the last prime's residues, which with a carry come from the words that job 0 overwrites).
     const bool no_tail = a.no_tail != 0;                                       // test / tuning switch
     int main_blocks = (int)blocks, tail_jobs = 0;
     const int rest = c_tiles % 8;
-    if (!no_tail && rest != 0 && c_tiles >= 8 && m_block == m_tiles && a.mod_num >= 8 && !a.raw_all) {
+    if (!no_tail && rest != 0 && c_tiles >= 8 && m_block == m_tiles && a.mod_num >= 8 && !a.raw_all && !a.carry) {
         tail_jobs = 4;
         main_blocks = (c_tiles / 8) * 8 * m_tiles;
         blocks = (unsigned)main_blocks + (unsigned)(rest * m_tiles * tail_jobs);
     }
-    hipLaunchKernelGGL((ppmm_mfma_kernel<DW, 8, 3, DC>), dim3(blocks), dim3(512), 0, stream, a, (const int8_t*)bdig, c_tiles, m_block, main_blocks, tail_jobs);
+    bool carried = false;
+    if constexpr (DW == 3) {                                                   // slices have three digits
+        carried = a.carry != 0;
+        if (carried) hipLaunchKernelGGL((ppmm_mfma_kernel<3, 8, 3, DC, true>), dim3(blocks), dim3(512), 0, stream, a, (const int8_t*)bdig, c_tiles, m_block, main_blocks, tail_jobs);
+    }
+    if (!carried) hipLaunchKernelGGL((ppmm_mfma_kernel<DW, 8, 3, DC, false>), dim3(blocks), dim3(512), 0, stream, a, (const int8_t*)bdig, c_tiles, m_block, main_blocks, tail_jobs);
     CKKS_HIP_TRY(hipGetLastError());
     return CKKS_OK;
 }

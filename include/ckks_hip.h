@@ -358,7 +358,7 @@ int pcmm_decode_coeffs(pcmm_ctx* h, double* vals, const uint64_t* plain, uint64_
  * base-256 digits: residues in 5 digits (primes up to 0x7f7f7f7f80, i.e. the 36-bit sets) or in 7 digits (primes below 2^50, i.e.
  * the reference's own 49-bit ring-pack primes), and |trunc(W*scaler)| below the smallest prime.  One launch takes a plaintext
  * matrix of up to 4 digits (3 with the 7-digit residues); wider ones, such as the 46-bit entries that the reference's scaler
- * q1 * 2^49 / scale gives, run as two or three launches over slices of three digits and a combining pass, with the same result.
+ * q1 * 2^49 / scale gives, run as two or three launches over slices of three digits, each adding to the one above it, with the same result.
  * Anything else takes a one-output-per-lane kernel with 128-bit accumulation (pcmm_info "last_path" tells which ran). */
 int pcmm_ppmm(pcmm_ctx* h, const float* W_dev, const uint64_t* const* mlwe_ptrs_host, uint64_t* out_dev, int M,
               int Kin, int mod_num, double scaler);

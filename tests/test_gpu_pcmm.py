@@ -276,6 +276,32 @@ def test_ppmm_random_shapes_on_one_context(wide):
     assert widths >= ({1, 2, 3, 4, 6, 7} if wide else {1, 2, 3, 4, 5})
 
 
+@pytest.mark.parametrize("bits, slices", [(24, 1), (34, 2), (33, 2)])
+@pytest.mark.parametrize("M", [1, 128, 130])
+def test_ppmm_slices_at_eight_moduli(bits, slices, M):
+    """Plaintext matrices of several slices where a single one would run its remainder column panels as jobs by prime (at least eight moduli, a
+    number of panels that is no multiple of eight): every lower slice reads what the one above left in the output.  Rows at the edge of a tile,
+    the largest entries of both signs, residues 0 and q - 1."""
+    q = CFG2_Q[:8]
+    N1, Kin = 64, 65
+    pair, dev, orc, rank = make(10, N1, CFG2_Q[:9], CFG3_P[:1], [CFG3_P[0]], q)
+    C = (rank + 1) * N1
+    assert C // 64 >= 8 and (C // 64) % 8
+    scaler, amax = float(2 ** 20), (1 << bits) - 1
+    W = (np.random.default_rng(bits).integers(-amax, amax + 1, (M, Kin)) / scaler).astype(np.float32)
+    W[0, :2], W[-1, -2:] = np.float32(amax / scaler), np.float32(-amax / scaler)
+    mlwe = [limbs_uniform(300 + n, q, 1, C)[0] for n in range(Kin)]
+    for j in range(8):
+        mlwe[0][j][:], mlwe[Kin - 1][j][:], mlwe[3][j][::2] = q[j] - 1, q[j] - 1, 0
+    want = np.zeros((M, 8, C), dtype=np.uint64)
+    orc.PPMM(W, [m.reshape(-1) for m in mlwe], want.reshape(-1), M, Kin, 8, scaler)
+    dout = DeviceBuffer(want.nbytes)
+    for _ in range(2):                                                    # the output still holds the first call's result
+        dev.PPMM(DeviceBuffer.from_numpy(W), [to_dev(m) for m in mlwe], dout, M, Kin, N1, Kin, 8, scaler)
+        assert dev.pcmm_context.info("last_path") == 1 and dev.pcmm_context.info("last_slices") == slices
+        assert np.array_equal(from_dev(dout, want.shape), want)
+
+
 def test_ppmm_reference_shape_50bit_primes():
     """The reference's own shape: two 50-bit ring-pack primes {q0, q1}, p_ringpack = {p_last}
     (test_rlwe_decomp.cu:36-49), scaler = q1 * 2^49 / scale (PPMM_kernel.cuh:283-284).  Residues of up to 50 bits take the MFMA
